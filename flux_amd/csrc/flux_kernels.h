@@ -156,6 +156,15 @@ __host__ __device__ constexpr int64_t split_partials_floats(int64_t m, int64_t n
     return kSplitBlocksK * m * n + kSplitBlocksK * m;
 }
 
+// GEMMs on three-limb bf16 products (prefill_limb_kernels.hip): block rows (256, 128 or 64 of
+// 128 columns) and K parts; parts > 1 leave that many partial planes in args.split_partials.
+struct LimbPlan {
+    int rows;
+    int parts;
+};
+LimbPlan limb_plan(const GemmArgs& args, int max_parts, bool fused_reduce);
+hipError_t launch_limb_gemm(const GemmArgs& args, GemmEpilogue epilogue, const LimbPlan& plan, hipStream_t stream);
+
 hipError_t launch_gemm(const GemmArgs& args, GemmEpilogue epilogue, hipStream_t stream);
 // epilogue(rmsnorm(A) * W^T): args.a holds the raw rows; `scratch` ([M, K]) receives the
 // normalized rows when the norm cannot be folded into the GEMM.
