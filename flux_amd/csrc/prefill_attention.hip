@@ -1,9 +1,8 @@
-// gfx950 causal GQA prefill attention on FP32 MFMA: one block per (128-query tile, query head,
-// key chunk), chunk partials merged by a second kernel; prompts up to 512 tokens take one block
-// per 32-query tile and head.
+// gfx950 causal GQA prefill attention (csrc/streaming_prefill_gqa/streaming_prefill_gqa_cuda.cu:
+// online softmax over K/V tiles in shared memory, no score materialisation).
 #include "flux_common.h"
 #include "flux_kernels.h"
-#include "prefill_common.h"
+#include "prefill_limb.h"
 
 #include <cmath>
 #include <type_traits>
@@ -12,43 +11,49 @@ namespace flux {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Causal GQA prefill attention on v_mfma_f32_32x32x2f32.
+// Causal GQA prefill attention on three-limb bf16 products (prefill_limb.h).
 //
 // Block = (128-query tile, query head, chunk of at most attn_chunk_tiles(seq) 64-key tiles);
-// 4 waves x 32 queries.  Per 64-key tile a wave computes S^T = K Q^T as two 32x32
-// tiles (32 MFMAs each: instruction s pairs dims s and s + 32), then
-// O^T += V^T P^T (16 MFMAs per 32 keys and 32-dim half): the S^T accumulator of a
-// lane is exactly the B operand of the PV product, so P never leaves registers.
-// O^T rows are dims 2i + db (db = 0, 1), so a lane's two V operands of one key are
-// adjacent floats.  Q is pre-scaled by scale * log2(e) so scores are already in
-// exp2 units.
+// 4 waves x 32 queries.  attention_limbs_kernel first splits the layer's K and V into limb
+// planes in MFMA operand order.  Per 64-key tile a wave computes S^T = K Q^T as two 32 x 32 tiles
+// (24 MFMAs each), then O^T += V^T P^T (12 MFMAs per 16 keys): a lane's S^T values are, in order,
+// the values of its B operand of the PV product, so P is split in registers and never leaves them.
+// Q is pre-scaled by scale * log2(e), so scores are already in exp2 units.
 //
-// K/V tiles stream HBM -> LDS with global_load_lds: one K buffer, refilled with the
+// K/V planes stream HBM -> LDS with global_load_lds: one K buffer, refilled with the
 // next tile as soon as every wave has finished its S^T, and two V buffers, the
 // next tile's copied while this tile's is read.  Each buffer is its own LDS
-// variable, so reads of one never wait on copies into another.  Three blocks fit a
-// CU (49 KB of LDS, at most 168 VGPRs), i.e. three waves per SIMD.
+// variable, so reads of one never wait on copies into another.  Two blocks fit a
+// CU (74 KB of LDS, 198 VGPRs), i.e. two waves per SIMD, one in its softmax while the other
+// multiplies.
 //
 // A query tile's keys are split into chunks of attn_chunk_tiles(seq) tiles: about one
 // block slot's even share of the causal work, so short prompts still spread over the device,
-// and at most kMaxChunkTiles (1024 keys) for long ones.  A tile with one
+// and at most kMaxChunkTiles (2048 keys) for long ones.  A tile with one
 // chunk writes its rows directly, longer ones write (o, m, l) partials that
 // prefill_attention_merge_kernel combines
-// (csrc/streaming_prefill_gqa/streaming_prefill_gqa_cuda.cu splits the keys into
+// (csrc/streaming_prefill_gqa/streaming_prefill_gqa_cuda.cu:43-460 splits the keys into
 // partitions and merges them the same way).  Items (query tile, chunk) are
 // launched longest first so the tail of the grid is short chunks.
 //
-// A wave raises its issue priority (s_setprio 1) for its QK and PV MFMA blocks and drops it
-// for the softmax: the other two waves of the SIMD then run their softmax and LDS work in
-// the gaps of its MFMA stream rather than delaying it (8192 tokens 35.21 → 35.08 ms; the
-// same around the GEMM kernels' MFMAs was slower).  Priority orders issue only; every wave
-// still reaches every barrier.
+// A wave raises its issue priority (s_setprio 1) for its MFMA blocks and drops it for the
+// softmax: the SIMD's other wave then runs its softmax and LDS work in the gaps of its MFMA
+// stream rather than delaying it.  Priority orders issue only; every wave still reaches every
+// barrier.
+//
+// Bound by power, as the limb GEMMs: 8192 tokens 632 -> 405 us with the planes and the merge
+// (191 TFLOP/s of float32 products, 1.15 PFLOP/s of bf16), 4096: 185 -> 117, 2048: 64 -> 47,
+// 1024: 30.5 -> 26.8; the error against 64 bits at 8000 tokens 4.3e-7 -> 1.7e-7.  Blocks whose
+// values limbs cannot hold, and prompts below kLimbAttnMinSeq, take the float32 instruction
+// (attention_item_f32).
 constexpr int kQTile = 128;
 constexpr int kKTile = 64;
 constexpr int kAttnThreads = 256;
-constexpr int kMaxChunkTiles = 16;  // 1024 keys: 24 (1536) measured 1.5% slower at 8192 tokens, 12 / 14 0.1%
+// Shorter prompts pay more for splitting K and V than they gain (832 tokens: 23.3 against 21.6 us).
+constexpr int64_t kLimbAttnMinSeq = 897;
+constexpr int kMaxChunkTiles = 32;  // 2048 keys: 16 measured 411 us at 8192 tokens and 128 at 4096, 24 411 and 117, 32 405 and 117
 constexpr int kPartialRow = kHeadDim + 4;  // o[64], m, l, 2 words of padding (16-byte rows)
-constexpr int kMergeMaxChunks = 16;        // >= the chunks of any query tile up to kMaxCapacity
+constexpr int kMergeMaxChunks = 16;       // >= the chunks of any query tile up to kMaxCapacity
 constexpr int kKVTileFloats = kKTile * kHeadDim;
 
 __host__ __device__ __forceinline__ int64_t attn_q_tiles(int64_t seq) { return (seq + kQTile - 1) / kQTile; }
@@ -57,13 +62,12 @@ __host__ __device__ __forceinline__ int64_t attn_key_tiles(int64_t seq, int64_t 
     return last / kKTile + 1;
 }
 // Key tiles per chunk: the 9 heads' causal tile steps (query tile qt walks 2 (qt + 1)
-// key tiles) divided over the device's 768 block slots (256 CUs x 3 resident blocks),
+// key tiles) divided over the device's 512 block slots (256 CUs x 2 resident blocks),
 // rounded up to an even count in [2, kMaxChunkTiles].  Even, because each query tile adds
-// two key tiles.  (Dividing over 256, 512, 1024 or 1536 instead measured slower at 2048 to
-// 4096 tokens.)
+// two key tiles.  (Dividing over 768 instead: 52.6 against 46.9 us at 2048 tokens.)
 __host__ __device__ __forceinline__ int64_t attn_chunk_tiles(int64_t seq) {
     const int64_t q = attn_q_tiles(seq);
-    const int64_t share = (kQHeads * q * (q + 1) + 767) / 768;
+    const int64_t share = (kQHeads * q * (q + 1) + 511) / 512;
     const int64_t even = (share + 1) / 2 * 2;
     return even < 2 ? 2 : (even > kMaxChunkTiles ? kMaxChunkTiles : even);
 }
@@ -132,19 +136,14 @@ constexpr int kKTileWords = kKTile * kKRow;           // 4352
 constexpr int kKCopies = kKTileWords / 256;           // 17 global_load_lds of 1 KB
 constexpr int kVCopies = kKVTileFloats / 256;         // 16
 
-__global__ void __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(3)))
-prefill_attention_kernel(const float* __restrict__ q, const float* __restrict__ key_cache,
-                         const float* __restrict__ value_cache, int64_t seq, int64_t capacity, float scale,
-                         float* __restrict__ workspace, float* __restrict__ out_rows) {
-    __shared__ __align__(16) float ks[kKTileWords];
-    __shared__ __align__(16) float v0s[kKVTileFloats];
-    __shared__ __align__(16) float v1s[kKVTileFloats];
-
+// One block's item on the float32 instruction, for values that limbs cannot hold.
+__device__ __forceinline__ void attention_item_f32(const float* __restrict__ q, const float* __restrict__ key_cache,
+                                                const float* __restrict__ value_cache, int64_t seq, int64_t capacity,
+                                                float scale, float* __restrict__ workspace,
+                                                float* __restrict__ out_rows, int h, int64_t qt, int64_t chunk,
+                                                float* ks, float* v0s, float* v1s) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int h = static_cast<int>(blockIdx.x % kQHeads);
-    int64_t qt, chunk;
-    attn_item(seq, blockIdx.x / kQHeads, qt, chunk);
     const int g = h / kGroup;
     const int64_t qw0 = qt * kQTile + 32 * wave;  // first query of this wave
     const int col = lane & 31;
@@ -361,6 +360,313 @@ prefill_attention_kernel(const float* __restrict__ q, const float* __restrict__ 
     if (!single && half == 0) *reinterpret_cast<float2*>(dst + kHeadDim) = make_float2(m_run, l_run);  // m in log2 units
 }
 
+// Prompts below kLimbAttnMinSeq: every block on the float32 instruction.
+__global__ void __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(3)))
+prefill_attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ key_cache,
+                             const float* __restrict__ value_cache, int64_t seq, int64_t capacity, float scale,
+                             float* __restrict__ workspace, float* __restrict__ out_rows) {
+    __shared__ __align__(16) float ks[kKTileWords];
+    __shared__ __align__(16) float v0s[kKVTileFloats];
+    __shared__ __align__(16) float v1s[kKVTileFloats];
+    int64_t qt, chunk;
+    attn_item(seq, blockIdx.x / kQHeads, qt, chunk);
+    attention_item_f32(q, key_cache, value_cache, seq, capacity, scale, workspace, out_rows,
+                       static_cast<int>(blockIdx.x % kQHeads), qt, chunk, ks, v0s, v1s);
+}
+
+// Limb planes of one layer's keys and values, so that the attention blocks copy MFMA operands
+// instead of splitting every tile again.  Per KV head and 64-key tile, 24 KB of K:
+// [key half][16-dim step][limb][dims 0-7 | 8-15][32 keys] x 8 values (16 bytes), and 24 KB of V:
+// [key half][step][dim half][limb][lane half][32 dims] x 8 values, whose slot e holds key
+// 8 (2 step + e / 4) + 4 (lane half) + e % 4 of the half: the keys whose probabilities a lane
+// holds after S^T.  Block (KV head, tile); rows past the prompt repeat its last row (masked).
+// flags[block] tells that a value of the tile is infinite or above the largest bf16.
+constexpr int kLimbTile = kKTile * kHeadDim * 2 * kLimbs;  // bytes of one K or V tile: 24576
+
+__device__ __forceinline__ bool too_large(const float (&v)[8]) {
+    float m = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) track_max(m, v[e], v[e + 1]);
+    return !(m <= kLimbMax);
+}
+
+__device__ __forceinline__ void store_limbs(char* at, const float (&v)[8]) {
+    const Limbs8 l = split8(f32x4{v[0], v[1], v[2], v[3]}, f32x4{v[4], v[5], v[6], v[7]});
+#pragma unroll
+    for (int j = 0; j < kLimbs; ++j) *reinterpret_cast<u32x4*>(at + 1024 * j) = l.limb[j];
+}
+
+__global__ void __launch_bounds__(256) attention_limbs_kernel(const float* __restrict__ key_cache,
+                                                              const float* __restrict__ value_cache, int64_t seq,
+                                                              int64_t capacity, char* __restrict__ k_planes,
+                                                              char* __restrict__ v_planes, int* __restrict__ flags) {
+    const int tiles = static_cast<int>((seq + kKTile - 1) / kKTile);
+    const int g = static_cast<int>(blockIdx.x) / tiles;
+    const int64_t key0 = static_cast<int64_t>(blockIdx.x % tiles) * kKTile;
+    const float* kg = key_cache + static_cast<int64_t>(g) * capacity * kHeadDim;
+    const float* vg = value_cache + static_cast<int64_t>(g) * capacity * kHeadDim;
+    char* kp = k_planes + static_cast<int64_t>(blockIdx.x) * kLimbTile;
+    char* vp = v_planes + static_cast<int64_t>(blockIdx.x) * kLimbTile;
+    bool large = false;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int u = static_cast<int>(threadIdx.x) + 256 * i;
+        float v[8];
+        const int key = u >> 3, part = u & 7;  // eight lanes per key row
+        const int64_t row = key0 + key < seq ? key0 + key : seq - 1;
+        *reinterpret_cast<f32x4*>(v) = *reinterpret_cast<const f32x4*>(kg + row * kHeadDim + 8 * part);
+        *reinterpret_cast<f32x4*>(v + 4) = *reinterpret_cast<const f32x4*>(kg + row * kHeadDim + 8 * part + 4);
+        large |= too_large(v);
+        store_limbs(kp + ((key >> 5) * 4 + (part >> 1)) * 3072 + (part & 1) * 512 + (key & 31) * 16, v);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int u = static_cast<int>(threadIdx.x) + 256 * i;
+        float v[8];
+        const int dim = u & 63, half = (u >> 6) & 1, step = u >> 7;  // step: 16-key group of the tile
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int64_t key = key0 + 16 * step + 8 * (e >> 2) + 4 * half + (e & 3);
+            v[e] = vg[(key < seq ? key : seq - 1) * kHeadDim + dim];
+        }
+        large |= too_large(v);
+        store_limbs(vp + (step * 2 + (dim >> 5)) * 3072 + half * 512 + (dim & 31) * 16, v);
+    }
+    const int any = __syncthreads_or(large);
+    if (threadIdx.x == 0) flags[blockIdx.x] = any;
+}
+
+__global__ void __launch_bounds__(kAttnThreads, 2)
+prefill_attention_kernel(const float* __restrict__ q, const float* __restrict__ key_cache,
+                         const float* __restrict__ value_cache, const char* __restrict__ k_planes,
+                         const char* __restrict__ v_planes, const int* __restrict__ flags, int64_t seq,
+                         int64_t capacity, float scale, float* __restrict__ workspace, float* __restrict__ out_rows) {
+    __shared__ __align__(16) char ks[kLimbTile];
+    __shared__ __align__(16) char v0s[kLimbTile];
+    __shared__ __align__(16) char v1s[kLimbTile];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = static_cast<int>(blockIdx.x % kQHeads);
+    int64_t qt, chunk;
+    attn_item(seq, blockIdx.x / kQHeads, qt, chunk);
+    const int g = h / kGroup;
+    const int64_t qw0 = qt * kQTile + 32 * wave;  // first query of this wave
+    const int col = lane & 31;
+    const int half = lane >> 5;
+    const int64_t my_q = qw0 + col;
+    const int64_t tiles = (seq + kKTile - 1) / kKTile;
+    const int64_t k_tiles = attn_key_tiles(seq, qt);
+    const int64_t chunk_tiles = attn_chunk_tiles(seq);
+    const int64_t kt_begin = chunk * chunk_tiles;
+    const int64_t kt_end = kt_begin + chunk_tiles < k_tiles ? kt_begin + chunk_tiles : k_tiles;
+
+    // B operand of S^T = K Q^T: the limbs of Q[my_q][16 step + 8 half ..] * scale * log2(e).
+    u32x4 qreg[4][kLimbs];
+    {
+        const int64_t r = my_q < seq ? my_q : seq - 1;
+        const float* qp = q + (static_cast<int64_t>(h) * seq + r) * kHeadDim + 8 * half;
+        const float s2 = scale * kLog2e;
+        bool large = false;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const f32x4 lo = *reinterpret_cast<const f32x4*>(qp + 16 * t) * s2;
+            const f32x4 hi = *reinterpret_cast<const f32x4*>(qp + 16 * t + 4) * s2;
+            const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            large |= too_large(v);
+            const Limbs8 l = split8(lo, hi);
+#pragma unroll
+            for (int j = 0; j < kLimbs; ++j) qreg[t][j] = l.limb[j];
+        }
+        if (kt_begin + lane < kt_end) large |= flags[g * tiles + kt_begin + lane] != 0;
+        if (__syncthreads_or(large)) {
+            attention_item_f32(q, key_cache, value_cache, seq, capacity, scale, workspace, out_rows, h, qt, chunk,
+                               reinterpret_cast<float*>(ks), reinterpret_cast<float*>(v0s),
+                               reinterpret_cast<float*>(v1s));
+            return;
+        }
+    }
+
+    // Copies of key tile kt: 24 of 1 KB each for K and V, wave w issues w, w + 4, ...
+    const char* kg = k_planes + static_cast<int64_t>(g) * tiles * kLimbTile + 16 * lane;
+    const char* vg = v_planes + static_cast<int64_t>(g) * tiles * kLimbTile + 16 * lane;
+    auto issue = [&](const char* planes, char* buf, int64_t kt) {
+#pragma unroll
+        for (int j = 0; j < kLimbTile / 4096; ++j) {
+            const int i = wave + 4 * j;
+            __builtin_amdgcn_global_load_lds(reinterpret_cast<const unsigned*>(planes + kt * kLimbTile + 1024 * i),
+                                             reinterpret_cast<unsigned*>(buf + 1024 * i), 16, 0, 0);
+        }
+    };
+
+    // O^T and its small limb products (prefill_limb.h), summed apart so that only the products
+    // of the leading limbs are rounded at the size of the result.
+    f32x16 o_acc[2], o_low[2];
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o_acc[db][r] = o_low[db][r] = 0.0f;
+    float m_run = -INFINITY;
+    float l_run = 0.0f;
+
+    const int seq32 = static_cast<int>(seq);
+    const int qw = static_cast<int>(qw0);
+    const int q_me = static_cast<int>(my_q);
+    // QK of 32 keys: the small products of all 64 dims first, those of the leading limbs last.
+    auto qk = [&](int kb, f32x16& c) {
+        const char* kp = ks + kb * 4 * 3072 + 16 * lane;
+        u32x4 lead[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            lead[t] = *reinterpret_cast<const u32x4*>(kp + 3072 * t);
+            const u32x4 k1 = *reinterpret_cast<const u32x4*>(kp + 3072 * t + 1024);
+            const u32x4 k2 = *reinterpret_cast<const u32x4*>(kp + 3072 * t + 2048);
+            c = mfma_bf16(k2, qreg[t][0], c);
+            c = mfma_bf16(lead[t], qreg[t][2], c);
+            c = mfma_bf16(k1, qreg[t][1], c);
+            c = mfma_bf16(k1, qreg[t][0], c);
+            c = mfma_bf16(lead[t], qreg[t][1], c);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) c = mfma_bf16(lead[t], qreg[t][0], c);
+    };
+    // One key tile: S^T from the K tile, an LDS barrier after which the K buffer is
+    // refilled with the next tile, then softmax and O^T += V^T P^T from this tile's
+    // V buffer.  Waves whose queries all precede the tile skip the math but not the
+    // barriers.
+    auto tile = [&](const char* vs, int64_t kt, int64_t kt_next) {
+        const int k0 = static_cast<int>(kt) * kKTile;
+        const bool active = k0 <= qw + 31;
+        const bool need_mask = k0 + kKTile - 1 > qw || k0 + kKTile > seq32;
+        const bool live1 = k0 + 32 <= qw + 31;  // second 32-key half visible to some query
+        f32x16 s_acc[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s_acc[kb][r] = 0.0f;
+        __builtin_amdgcn_s_setprio(1);  // the MFMA block (see above the kernel)
+        if (active) qk(0, s_acc[0]);
+        if (live1) qk(1, s_acc[1]);
+        __builtin_amdgcn_s_setprio(0);
+        lds_barrier();  // every wave is done with the K tile
+        issue(kg, ks, kt_next);
+        if (!active) return;
+        // Lane holds keys k0 + 32 kb + 8 (r / 4) + 4 half + r % 4 of query my_q.
+        if (!live1) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s_acc[1][r] = -INFINITY;
+        }
+        if (need_mask) {
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int key = k0 + 32 * kb + 8 * (r >> 2) + 4 * half + (r & 3);
+                    s_acc[kb][r] = (key <= q_me && key < seq32) ? s_acc[kb][r] : -INFINITY;
+                }
+            }
+        }
+        float tile_max = -INFINITY;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) tile_max = fmaxf(tile_max, s_acc[kb][r]);
+        tile_max = halves_max(tile_max);
+        const float m_new = fmaxf(m_run, tile_max);  // finite: the first key of a chunk precedes every query
+        const float alpha = fast_exp2(m_run - m_new);
+        float psum = 0.0f;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float p = fast_exp2(s_acc[kb][r] - m_new);
+                s_acc[kb][r] = p;
+                psum += p;
+            }
+        }
+        psum = halves_sum(psum);
+        l_run = l_run * alpha + psum;
+        m_run = m_new;
+        // alpha is exactly 1 where the running max did not move: skip the rescale
+        // when that holds for every lane (multiplying by 1 would not change a bit).
+        if (__any(alpha != 1.0f)) {
+#pragma unroll
+            for (int db = 0; db < 2; ++db) {
+                o_acc[db] *= alpha;
+                o_low[db] *= alpha;
+            }
+        }
+        const char* vp = vs + 16 * lane;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            if (kb == 1 && !live1) continue;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const f32x16& s = s_acc[kb];
+                const Limbs8 p = split8(f32x4{s[8 * t], s[8 * t + 1], s[8 * t + 2], s[8 * t + 3]},
+                                        f32x4{s[8 * t + 4], s[8 * t + 5], s[8 * t + 6], s[8 * t + 7]});
+                u32x4 v[2][kLimbs];
+#pragma unroll
+                for (int db = 0; db < 2; ++db)
+#pragma unroll
+                    for (int l = 0; l < kLimbs; ++l)
+                        v[db][l] =
+                            *reinterpret_cast<const u32x4*>(vp + ((kb * 2 + t) * 2 + db) * 3072 + 1024 * l);
+                __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+                for (int db = 0; db < 2; ++db) o_low[db] = mfma_bf16(v[db][2], p.limb[0], o_low[db]);
+#pragma unroll
+                for (int db = 0; db < 2; ++db) o_low[db] = mfma_bf16(v[db][0], p.limb[2], o_low[db]);
+#pragma unroll
+                for (int db = 0; db < 2; ++db) o_low[db] = mfma_bf16(v[db][1], p.limb[1], o_low[db]);
+#pragma unroll
+                for (int db = 0; db < 2; ++db) o_low[db] = mfma_bf16(v[db][1], p.limb[0], o_low[db]);
+#pragma unroll
+                for (int db = 0; db < 2; ++db) o_low[db] = mfma_bf16(v[db][0], p.limb[1], o_low[db]);
+#pragma unroll
+                for (int db = 0; db < 2; ++db) o_acc[db] = mfma_bf16(v[db][0], p.limb[0], o_acc[db]);
+                __builtin_amdgcn_s_setprio(0);
+            }
+        }
+    };
+
+    issue(kg, ks, kt_begin);
+    issue(vg, v0s, kt_begin);
+    __builtin_amdgcn_s_waitcnt(0);
+    lds_barrier();
+    for (int64_t kt = kt_begin; kt < kt_end; kt += 2) {
+        const int64_t n1 = kt + 1 < kt_end ? kt + 1 : kt_end - 1;
+        issue(vg, v1s, n1);
+        tile(v0s, kt, n1);
+        __builtin_amdgcn_s_waitcnt(0);  // this wave's copies of tile kt + 1 have landed
+        lds_barrier();
+        if (kt + 1 < kt_end) {
+            const int64_t n2 = kt + 2 < kt_end ? kt + 2 : kt_end - 1;
+            issue(vg, v0s, n2);
+            tile(v1s, kt + 1, n2);
+            __builtin_amdgcn_s_waitcnt(0);
+            lds_barrier();
+        }
+    }
+
+    // O^T accumulator: lane holds dims 32 db + 8 (r / 4) + 4 half + r % 4 of query my_q.
+    if (my_q >= seq) return;
+    const bool single = attn_chunks(seq, qt) == 1;
+    const float inv = single ? 1.0f / l_run : 1.0f;
+    float* dst = single ? out_rows + my_q * kHidden + h * kHeadDim
+                        : workspace + (attn_partial_slot(seq, qt, h, chunk) * kQTile + (my_q - qt * kQTile)) * kPartialRow;
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+            f32x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = (o_acc[db][r + e] + o_low[db][r + e]) * inv;
+            *reinterpret_cast<f32x4*>(dst + 32 * db + 2 * r + 4 * half) = o;
+        }
+    if (!single && half == 0) *reinterpret_cast<float2*>(dst + kHeadDim) = make_float2(m_run, l_run);  // m in log2 units
+}
+
 // Combines the chunk partials of query tiles with more than one chunk.  Block
 // ((qt - attn_long_tile(seq)) * 9 + h) * 8 + row group; thread t -> row 16 * group + t / 16,
 // dims 4 (t % 16) .. + 3.  All chunk loads of a thread are issued before the combine.
@@ -567,11 +873,19 @@ prefill_attention_small_kernel(const float* __restrict__ q, const float* __restr
 
 }  // namespace
 
-size_t prefill_attention_workspace_floats(int64_t seq) {
-    if (seq <= kSmallAttnMaxSeq) return 0;  // prefill_attention_small_kernel keeps its partials in LDS
+// Floats of the split-key partials (a multiple of 4).
+static int64_t attn_partial_floats(int64_t seq) {
     const int64_t long_tiles = attn_q_tiles(seq) - attn_long_tile(seq);
     if (long_tiles <= 0 || attn_max_chunks(seq) <= 1) return 0;
-    return static_cast<size_t>(long_tiles * kQHeads * attn_max_chunks(seq) * kQTile * kPartialRow);
+    return long_tiles * kQHeads * attn_max_chunks(seq) * kQTile * kPartialRow;
+}
+
+size_t prefill_attention_workspace_floats(int64_t seq) {
+    if (seq <= kSmallAttnMaxSeq) return 0;  // prefill_attention_small_kernel keeps its partials in LDS
+    if (seq < kLimbAttnMinSeq) return static_cast<size_t>(attn_partial_floats(seq));
+    // Partials, the limb planes of K and V, and one flag per key tile.
+    const int64_t tiles = kKVHeads * ((seq + kKTile - 1) / kKTile);
+    return static_cast<size_t>(attn_partial_floats(seq) + tiles * (2 * kLimbTile / 4) + (tiles + 3) / 4 * 4);
 }
 
 hipError_t launch_prefill_attention(const float* q, const float* key_cache, const float* value_cache, int64_t seq,
@@ -586,10 +900,25 @@ hipError_t launch_prefill_attention(const float* q, const float* key_cache, cons
         return hipGetLastError();
     }
     if (attn_max_chunks(seq) > kMergeMaxChunks) return hipErrorInvalidValue;
-    const int64_t blocks = attn_items(seq) * kQHeads;
-    hipLaunchKernelGGL(prefill_attention_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kAttnThreads), 0, stream, q,
-                       key_cache, value_cache, seq, capacity, scale, workspace, out_rows);
-    hipError_t st = hipGetLastError();
+    const dim3 blocks(static_cast<unsigned>(attn_items(seq) * kQHeads));
+    hipError_t st = hipSuccess;
+    if (seq < kLimbAttnMinSeq) {
+        hipLaunchKernelGGL(prefill_attention_f32_kernel, blocks, dim3(kAttnThreads), 0, stream, q, key_cache,
+                           value_cache, seq, capacity, scale, workspace, out_rows);
+        st = hipGetLastError();
+    } else {
+        const int64_t tiles = kKVHeads * ((seq + kKTile - 1) / kKTile);
+        char* k_planes = reinterpret_cast<char*>(workspace + attn_partial_floats(seq));
+        char* v_planes = k_planes + tiles * kLimbTile;
+        int* flags = reinterpret_cast<int*>(v_planes + tiles * kLimbTile);
+        hipLaunchKernelGGL(attention_limbs_kernel, dim3(static_cast<unsigned>(tiles)), dim3(256), 0, stream, key_cache,
+                           value_cache, seq, capacity, k_planes, v_planes, flags);
+        st = hipGetLastError();
+        if (st != hipSuccess) return st;
+        hipLaunchKernelGGL(prefill_attention_kernel, blocks, dim3(kAttnThreads), 0, stream, q, key_cache, value_cache,
+                           k_planes, v_planes, flags, seq, capacity, scale, workspace, out_rows);
+        st = hipGetLastError();
+    }
     if (st != hipSuccess) return st;
     const int64_t long_tiles = attn_q_tiles(seq) - attn_long_tile(seq);
     if (long_tiles > 0 && attn_max_chunks(seq) > 1) {

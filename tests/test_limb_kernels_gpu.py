@@ -69,3 +69,63 @@ def test_limb_linear_keeps_float32_range(gpu_device):
     torch.testing.assert_close(c[700].double(), a[700].double() @ w.double().T, rtol=0, atol=1e-42 * k)
     rows = [r for r in range(m) if r not in (3, 4, 5, 6, 700)]
     torch.testing.assert_close(c[rows].double(), a[rows].double() @ w.double().T, rtol=1e-4, atol=1e-4)
+
+
+def _attention(q, k, v, device):
+    lib = _native.load()
+    seq = q.shape[1]
+    need = ctypes.c_int64()
+    _native.check(lib.flux_prefill_attention_workspace_bytes(seq, ctypes.byref(need)))
+    q, k, v = q.to(device), k.to(device), v.to(device)
+    workspace = torch.empty(max(1, need.value // 4), device=device)
+    out = torch.empty(seq, 576, device=device)
+    _native.check(lib.flux_prefill_attention_f32(q.data_ptr(), k.data_ptr(), v.data_ptr(), seq, k.shape[1], 0.125,
+                                                 workspace.data_ptr(), out.data_ptr(),
+                                                 _native.current_stream(device)))
+    torch.cuda.synchronize()
+    return out.cpu().view(seq, 9, 64).transpose(0, 1).double()
+
+
+def _attention64(q, k, v):
+    seq = q.shape[1]
+    k, v = (t.double()[:, :seq].repeat_interleave(3, 0) for t in (k, v))
+    scores = q.double() @ k.transpose(1, 2) * 0.125
+    scores.masked_fill_(torch.ones(seq, seq, dtype=torch.bool).triu(1), float("-inf"))
+    return torch.softmax(scores, -1) @ v
+
+
+# 896 | 897: below and above the shortest limb prompt; 961: a last key tile of one row; 1153: a
+# last query tile of one row; 2400: chunks of 8 tiles, the last one partial.
+@pytest.mark.parametrize("seq", [896, 897, 961, 1153, 2400])
+def test_limb_attention_is_as_exact_as_float32(gpu_device, seq):
+    q, k, v = (_randn(h, seq + 7 * (h == 3), 64, seed=10 + i) for i, h in enumerate((9, 3, 3)))
+    want = _attention64(q, k, v)
+    got = _attention(q, k, v, gpu_device)
+    # Scores of 64 products and at most seq weights that sum to one: a relative 1e-6 is two units
+    # in the last place of float32 for every ninth of them.
+    assert float((got - want).norm() / want.norm()) < 1e-6
+    torch.testing.assert_close(got, want, rtol=2e-4, atol=2e-5)
+
+
+def test_limb_attention_keeps_float32_range(gpu_device):
+    # A key that no query can see (its score is -inf), one above the largest bf16 and a value that
+    # is infinite: the blocks that read them take the float32 instruction, the others do not.
+    seq = 1500
+    q, k, v = _randn(9, seq, 64, seed=20), _randn(3, seq, 64, seed=21), _randn(3, seq, 64, seed=22)
+    q[:, :, 0] = -q[:, :, 0].abs() - 0.1
+    k[0, 700, 0] = float("inf")
+    k[1, 3, 0] = 3.4e38
+    v[2, 1000, 5] = float("inf")
+    got = _attention(q, k, v, gpu_device)
+    seen = k.clone()
+    seen[0, 700] = 0.0
+    want = _attention64(q, k, v)
+    k0 = seen[0].double()
+    scores = q[:3].double() @ k0.T * 0.125
+    scores[:, :, 700] = float("-inf")
+    scores.masked_fill_(torch.ones(seq, seq, dtype=torch.bool).triu(1), float("-inf"))
+    want[:3] = torch.softmax(scores, -1) @ v[0].double()
+    torch.testing.assert_close(got[:6], want[:6], rtol=2e-4, atol=2e-5)
+    assert torch.all(got[6:, 1000:, 5] == float("inf"))
+    rest = [d for d in range(64) if d != 5]
+    torch.testing.assert_close(got[6:, :, rest], want[6:, :, rest], rtol=2e-4, atol=2e-5)
