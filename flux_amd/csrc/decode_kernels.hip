@@ -17,8 +17,8 @@
 // Per layer the phases are
 //   A  norm(h) -> packed QKV GEMV -> RoPE(q,k) -> K/V cache write   (480 waves)
 //   B  split-K GQA attention partials, one (KV head, position chunk) per WG
-//      (one chunk per 64 attended positions, at most 85 per KV head)
-//   B2 merge partials per query head (36 WGs: query head x 16 dims)
+//      (one chunk up to 128 attended positions, then one per 64, at most 85 per KV head)
+//   B2 merge partials per query head (36 WGs: query head x 16 dims; not with one chunk)
 //   C  o_proj GEMV + residual                                        (576 waves)
 //   D  norm(r) -> packed gate/up GEMV -> SwiGLU                      (1536 waves)
 //   E  down GEMV + residual                                          (576 waves)
@@ -50,6 +50,7 @@ __device__ __forceinline__ unsigned tid_opaque() {
 constexpr int kThreads = 512;
 constexpr int kWavesPerWG = kThreads / kWave;
 constexpr int kAttnRows = 224;            // attention rows per workgroup (LDS-resident K/V)
+constexpr int kSingleChunkRows = 128;     // attended positions that one workgroup per KV head takes whole
 constexpr int kLmBatch = 4;
 // A wait that has lasted this long (or its bound, if shorter) starts watching the
 // device error word (so one workgroup's timeout ends every other workgroup's wait at
@@ -591,26 +592,53 @@ __device__ __forceinline__ void attn_compute(const float* k_lds, const float* v_
         constexpr int kS = kGroup * kHeadDim;
         const float a0 = (src[0] + src[kS]) + (src[2 * kS] + src[3 * kS]);
         const float a1 = (src[4 * kS] + src[5 * kS]) + (src[6 * kS] + src[7 * kS]);
-        out.put(h, lane, a0 * f0 + a1 * f1);
-        if (lane == 0) {
-            out.put(h, kHeadDim, M);
-            out.put(h, kHeadDim + 1, red_ml[2 * kGroup + h * 2] * f0 + red_ml[2 * kGroup + h * 2 + 1] * f1);
-        }
+        out.put(h, lane, a0 * f0 + a1 * f1, M, red_ml[2 * kGroup + h * 2] * f0 + red_ml[2 * kGroup + h * 2 + 1] * f1);
     }
     __syncthreads();
     FLUX_ATTN_TRACE(3);
 }
 
 // ---------------------------------------------------------------------------
-// Partial output addressing: partial (g, c) has kGroup * 66 slots.
+// Outputs of attn_compute for query head h of the group: lane d holds o[d] (unnormalised), every
+// lane the maximum m and the sum l.  Partial (g, c) has kGroup * 66 slots.
 struct PartialPlainOut {
     float* p;
-    __device__ __forceinline__ void put(int h, int j, float v) const { p[h * (kHeadDim + 2) + j] = v; }
+    __device__ __forceinline__ void put(int h, int lane, float o, float m, float l) const {
+        float* slot = p + h * (kHeadDim + 2);
+        slot[lane] = o;
+        if (lane == 0) {
+            slot[kHeadDim] = m;
+            slot[kHeadDim + 1] = l;
+        }
+    }
 };
+// The partial's LL words, or, when one chunk holds every position, the finished head in every copy
+// of the merged vector.
 struct PartialLLOut {
-    uint64_t* p;
+    uint64_t* ll;  // the layer's parity block
+    int group;
+    int chunk;
+    int chunks;
     uint32_t epoch;
-    __device__ __forceinline__ void put(int h, int j, float v) const { ll_store(p + h * (kHeadDim + 2) + j, v, epoch); }
+    __device__ __forceinline__ void put(int h, int lane, float o, float m, float l) const {
+        // Read through an empty asm, so that nothing derived from it is held across the attention
+        // (0.3% per token at long contexts).
+        int single = chunks;
+        asm volatile("" : "+s"(single));
+        if (single == 1) {
+            const float v = o / l;
+            uint64_t* merged = ll + LLLayout::kAttnMerged + (group * kGroup + h) * kHeadDim + lane;
+#pragma unroll
+            for (int r = 0; r < LLLayout::kReplicas; ++r) ll_store(merged + r * LLLayout::kReplicaStride, v, epoch);
+            return;
+        }
+        uint64_t* slot = ll + LLLayout::kPartials + ((group * chunks + chunk) * kGroup + h) * (kHeadDim + 2);
+        ll_store(slot + lane, o, epoch);
+        if (lane == 0) {
+            ll_store(slot + kHeadDim, m, epoch);
+            ll_store(slot + kHeadDim + 1, l, epoch);
+        }
+    }
 };
 
 // Chunking of the attended positions [0, L) across `chunks` workgroups.
@@ -915,7 +943,12 @@ __global__ void __launch_bounds__(kThreads, 1) fused_decode_kernel(DecodeArgs ar
         // `chunks` (85 on 256 CUs, reached from 5377 positions on).  Short contexts then
         // merge a few partials instead of 85 mostly one-row ones (ctx 128: 0.457 -> 0.427 ms
         // per token, 1024: 0.472 -> 0.436; 64-row chunks measured faster than 32, 96 or 128).
-        const int want_chunks = static_cast<int>((attended + 63) >> 6);
+        // Up to kSingleChunkRows positions one workgroup per KV head takes them all and publishes
+        // the finished heads itself: no merge, no exchange of partials.  Its body takes as long as
+        // a 64-row chunk's (one pass of 128 rows); a second pass and the longer copy would cost
+        // what the merge does.  Per token: 8 positions 377 -> 329 us, 90: 386 -> 356, 128: 388 ->
+        // 375; at 160 positions it measured even, at 190 5% slower.
+        const int want_chunks = attended <= kSingleChunkRows ? 1 : static_cast<int>((attended + 63) >> 6);
         const int tchunks_token = __builtin_amdgcn_readfirstlane(want_chunks < chunks ? want_chunks : chunks);
         const float* emb_row = args.embedding + (token_ok ? token : 0) * kHidden;
 
@@ -1021,13 +1054,13 @@ __global__ void __launch_bounds__(kThreads, 1) fused_decode_kernel(DecodeArgs ar
                 FLUX_TRACE_POINT(3);
                 attn_compute(k_lds, v_lds, vec, static_cast<int>(end - begin), Lw.scale * kLog2e,
                              AttnScratch{attn_sp, attn_pl, red},
-                             PartialLLOut{ll + LLLayout::kPartials + (g * tchunks + c) * partial_stride, ep}
+                             PartialLLOut{ll, g, c, tchunks, ep}
                                  FLUX_TRACE_ARG);
             }
 
             FLUX_TRACE_POINT(4);
             // ---- B2: merge chunk partials; WG (h, quarter) handles 16 dims of query head h ----
-            if (wg < kQHeads * 4) {
+            if (wg < kQHeads * 4 && tchunks != 1) {
                 const int h = wg >> 2;
                 const int quarter = wg & 3;
                 const int g = h / kGroup;

@@ -595,3 +595,19 @@ def test_wait_timeout_reports_error_and_invalid_tokens(small_model):
     torch.cuda.synchronize()
     assert again[0].cpu().numpy().tolist() == record["tokens"].tolist()
     assert runtime.device_error() == 0
+
+
+def test_decode_across_the_single_chunk_limit(small_model):
+    """Teacher-forced decode from 126 to 131 attended positions and at 2: up to 128 one workgroup per
+    KV head attends all of them and publishes the finished heads, beyond that two or more chunks are
+    merged.  Each step's logits equal the native prefill's of the extended prompt."""
+    g = torch.Generator().manual_seed(128)
+    tokens = torch.randint(0, 128, (1, 131), generator=g).cuda()
+    for n_prompt, steps in ((1, 1), (125, 6)):
+        runtime = NativeSmolLM2Prefill.capture(small_model, tokens[:, :n_prompt], max_decode_steps=steps)
+        for step in range(steps):
+            decoded = runtime.replay(tokens[:, n_prompt + step:n_prompt + step + 1])[0, 0].float().cpu().clone()
+            reference = NativeSmolLM2Prefill.capture(small_model, tokens[:, :n_prompt + step + 1], max_decode_steps=0)
+            torch.testing.assert_close(decoded, reference.logits[0, 0].float().cpu(), atol=LOGIT_ATOL, rtol=LOGIT_RTOL,
+                                       msg=lambda m: f"{n_prompt} + {step}: {m}")
+        assert runtime.device_error() == 0
