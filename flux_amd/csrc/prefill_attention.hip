@@ -43,7 +43,7 @@ namespace {
 //
 // Bound by power, as the limb GEMMs: 8192 tokens 632 -> 405 us with the planes and the merge
 // (191 TFLOP/s of float32 products, 1.15 PFLOP/s of bf16), 4096: 185 -> 117, 2048: 64 -> 47,
-// 1024: 30.5 -> 26.8; the error against 64 bits at 8000 tokens 4.3e-7 -> 1.7e-7.  Blocks whose
+// 1024: 30.6 -> 27.5; the error against 64 bits at 8000 tokens 4.3e-7 -> 1.7e-7.  Blocks whose
 // values limbs cannot hold, and prompts below kLimbAttnMinSeq, take the float32 instruction
 // (attention_item_f32).
 constexpr int kQTile = 128;
@@ -53,7 +53,7 @@ constexpr int kAttnThreads = 256;
 constexpr int64_t kLimbAttnMinSeq = 897;
 constexpr int kMaxChunkTiles = 32;  // 2048 keys: 16 measured 411 us at 8192 tokens and 128 at 4096, 24 411 and 117, 32 405 and 117
 constexpr int kPartialRow = kHeadDim + 4;  // o[64], m, l, 2 words of padding (16-byte rows)
-constexpr int kMergeMaxChunks = 16;       // >= the chunks of any query tile up to kMaxCapacity
+constexpr int kMergeMaxChunks = 8;         // >= the chunks of any query tile up to kMaxCapacity
 constexpr int kKVTileFloats = kKTile * kHeadDim;
 
 __host__ __device__ __forceinline__ int64_t attn_q_tiles(int64_t seq) { return (seq + kQTile - 1) / kQTile; }
@@ -61,16 +61,27 @@ __host__ __device__ __forceinline__ int64_t attn_key_tiles(int64_t seq, int64_t 
     const int64_t last = (qt + 1) * kQTile - 1 < seq - 1 ? (qt + 1) * kQTile - 1 : seq - 1;
     return last / kKTile + 1;
 }
-// Key tiles per chunk: the 9 heads' causal tile steps (query tile qt walks 2 (qt + 1)
-// key tiles) divided over the device's 512 block slots (256 CUs x 2 resident blocks),
-// rounded up to an even count in [2, kMaxChunkTiles].  Even, because each query tile adds
-// two key tiles.  (Dividing over 768 instead: 52.6 against 46.9 us at 2048 tokens.)
-__host__ __device__ __forceinline__ int64_t attn_chunk_tiles(int64_t seq) {
+// Even number of key tiles that is one of `slots` even shares of the 9 heads' causal tile steps
+// (query tile qt walks 2 (qt + 1) key tiles), in [2, most].  Even, because each query tile adds
+// two key tiles.
+__host__ __device__ __forceinline__ int64_t attn_share_tiles(int64_t seq, int64_t slots, int64_t most) {
     const int64_t q = attn_q_tiles(seq);
-    const int64_t share = (kQHeads * q * (q + 1) + 511) / 512;
+    const int64_t share = (kQHeads * q * (q + 1) + slots - 1) / slots;
     const int64_t even = (share + 1) / 2 * 2;
-    return even < 2 ? 2 : (even > kMaxChunkTiles ? kMaxChunkTiles : even);
+    return even < 2 ? 2 : (even > most ? most : even);
 }
+// Key tiles per chunk: an even share of the device's 512 block slots (256 CUs x 2 resident blocks;
+// dividing over 768 instead: 52.6 against 46.9 us at 2048 tokens).  Up to 14 query tiles the chunks
+// are longer than that, so that partials and limb planes together fit the workspace of
+// prefill_attention_workspace_floats.
+__host__ __device__ __forceinline__ int64_t attn_chunk_tiles(int64_t seq) {
+    const int64_t share = attn_share_tiles(seq, 512, kMaxChunkTiles);
+    if (seq < kLimbAttnMinSeq) return share;
+    const int64_t q = attn_q_tiles(seq);
+    const int64_t least = q <= 12 ? 4 : (q <= 14 ? 6 : 2);
+    return share < least ? least : share;
+}
+
 __host__ __device__ __forceinline__ int64_t attn_chunks(int64_t seq, int64_t qt) {
     const int64_t ct = attn_chunk_tiles(seq);
     return (attn_key_tiles(seq, qt) + ct - 1) / ct;
@@ -880,12 +891,25 @@ static int64_t attn_partial_floats(int64_t seq) {
     return long_tiles * kQHeads * attn_max_chunks(seq) * kQTile * kPartialRow;
 }
 
+// Floats that the kernels use: the partials, and from kLimbAttnMinSeq on the limb planes of K and V
+// and one flag per key tile.
+static int64_t attn_used_floats(int64_t seq) {
+    const int64_t tiles = kKVHeads * ((seq + kKTile - 1) / kKTile);
+    return attn_partial_floats(seq) +
+           (seq < kLimbAttnMinSeq ? 0 : tiles * (2 * kLimbTile / 4) + (tiles + 3) / 4 * 4);
+}
+
+// The size callers are told: partials of chunks of an even share of 768 slots and at most 16 key
+// tiles, which covers what is used at every length (launch_prefill_attention checks it), so that
+// a workspace kept from an earlier version of the library still fits.
 size_t prefill_attention_workspace_floats(int64_t seq) {
     if (seq <= kSmallAttnMaxSeq) return 0;  // prefill_attention_small_kernel keeps its partials in LDS
-    if (seq < kLimbAttnMinSeq) return static_cast<size_t>(attn_partial_floats(seq));
-    // Partials, the limb planes of K and V, and one flag per key tile.
-    const int64_t tiles = kKVHeads * ((seq + kKTile - 1) / kKTile);
-    return static_cast<size_t>(attn_partial_floats(seq) + tiles * (2 * kLimbTile / 4) + (tiles + 3) / 4 * 4);
+    const int64_t ct = attn_share_tiles(seq, 768, 16);
+    const int64_t q_tiles = attn_q_tiles(seq);
+    const int64_t max_chunks = (attn_key_tiles(seq, q_tiles - 1) + ct - 1) / ct;
+    const int64_t long_tiles = q_tiles - ct * kKTile / kQTile;
+    if (long_tiles <= 0 || max_chunks <= 1) return 0;
+    return static_cast<size_t>(long_tiles * kQHeads * max_chunks * kQTile * kPartialRow);
 }
 
 hipError_t launch_prefill_attention(const float* q, const float* key_cache, const float* value_cache, int64_t seq,
@@ -899,7 +923,9 @@ hipError_t launch_prefill_attention(const float* q, const float* key_cache, cons
                            value_cache, seq, capacity, scale, out_rows);
         return hipGetLastError();
     }
-    if (attn_max_chunks(seq) > kMergeMaxChunks) return hipErrorInvalidValue;
+    if (attn_max_chunks(seq) > kMergeMaxChunks ||
+        attn_used_floats(seq) > static_cast<int64_t>(prefill_attention_workspace_floats(seq)))
+        return hipErrorInvalidValue;
     const dim3 blocks(static_cast<unsigned>(attn_items(seq) * kQHeads));
     hipError_t st = hipSuccess;
     if (seq < kLimbAttnMinSeq) {
@@ -922,14 +948,10 @@ hipError_t launch_prefill_attention(const float* q, const float* key_cache, cons
     if (st != hipSuccess) return st;
     const int64_t long_tiles = attn_q_tiles(seq) - attn_long_tile(seq);
     if (long_tiles > 0 && attn_max_chunks(seq) > 1) {
-        // Registers for at most 4, 8 or 16 chunks: fewer registers, more waves in flight.
+        // Registers for at most 4 or 8 chunks: fewer registers, more waves in flight.
         const dim3 grid(static_cast<unsigned>(long_tiles * kQHeads * (kQTile / (kAttnThreads / 16))));
-        const int64_t chunks = attn_max_chunks(seq);
-        if (chunks <= 4)
+        if (attn_max_chunks(seq) <= 4)
             hipLaunchKernelGGL(prefill_attention_merge_kernel<4>, grid, dim3(kAttnThreads), 0, stream, workspace, seq,
-                               out_rows);
-        else if (chunks <= 8)
-            hipLaunchKernelGGL(prefill_attention_merge_kernel<8>, grid, dim3(kAttnThreads), 0, stream, workspace, seq,
                                out_rows);
         else
             hipLaunchKernelGGL(prefill_attention_merge_kernel<kMergeMaxChunks>, grid, dim3(kAttnThreads), 0, stream,
