@@ -14,6 +14,7 @@ host.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import math
 from typing import Sequence
@@ -68,7 +69,10 @@ for _schema in SCHEMAS.values():
 # Helpers.
 
 def _check(condition, message: str) -> None:
-    torch._check(condition, lambda: message)
+    # torch._check costs 1 us, and an operator makes about ten checks: it is called for what is
+    # not plainly true, i.e. a failure or, under tracing, a symbolic condition.
+    if condition is not True:
+        torch._check(condition, lambda: message)
 
 
 def _grad_free(op: str, *tensors: torch.Tensor | None) -> None:
@@ -85,8 +89,19 @@ def _aliases(a: torch.Tensor, b: torch.Tensor) -> bool:
     return a.device == b.device and a.untyped_storage().data_ptr() == b.untyped_storage().data_ptr()
 
 
+_STRIDE_ARRAYS = {count: ctypes.c_int64 * count for count in (3, 4)}
+
+
 def _strides(tensor: torch.Tensor, count: int):
-    return _native.length_array([int(s) for s in tensor.stride()[:count]])
+    return _STRIDE_ARRAYS[count](*tensor.stride()[:count])
+
+
+_NO_SWITCH = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing to do where that device is current already."""
+    return _NO_SWITCH if device.index == torch.cuda.current_device() else torch.cuda.device(device)
 
 
 def _call(function: str, *args) -> None:
@@ -137,7 +152,7 @@ def _validate_rmsnorm_out(input, weight, epsilon, output) -> None:
 def _launch_rmsnorm(input, weight, epsilon, output) -> None:
     cols = int(input.shape[-1])
     _check(cols <= _RMSNORM_MAX_WIDTH, f"flux::rmsnorm: final dimension above {_RMSNORM_MAX_WIDTH} is unsupported")
-    with torch.cuda.device(input.device):
+    with _on(input.device):
         _call("flux_rmsnorm_f32", input.data_ptr(), weight.data_ptr(), output.data_ptr(), input.numel() // cols, cols,
               float(epsilon), _stream(input))
 
@@ -184,7 +199,7 @@ def _launch_residual_rmsnorm(hidden, residual, weight, epsilon, norm_out, residu
     cols = int(hidden.shape[-1])
     _check(cols <= _RMSNORM_MAX_WIDTH,
            f"flux::residual_rmsnorm: final dimension above {_RMSNORM_MAX_WIDTH} is unsupported")
-    with torch.cuda.device(hidden.device):
+    with _on(hidden.device):
         _call("flux_residual_rmsnorm_f32", hidden.data_ptr(), residual.data_ptr(), weight.data_ptr(),
               norm_out.data_ptr(), residual_out.data_ptr(), hidden.numel() // cols, cols, float(epsilon),
               _stream(hidden))
@@ -246,7 +261,7 @@ def _rope_cuda(query, key, cos, sin):
     query_out = torch.empty(query.shape, dtype=torch.float32, device=query.device)
     key_out = torch.empty(key.shape, dtype=torch.float32, device=key.device)
     batch, query_heads, seq, dim = (int(s) for s in query.shape)
-    with torch.cuda.device(query.device):
+    with _on(query.device):
         _call("flux_rope_f32", query.data_ptr(), key.data_ptr(), cos.data_ptr(), sin.data_ptr(), query_out.data_ptr(),
               key_out.data_ptr(), batch, query_heads, int(key.shape[1]), seq, dim, int(cos.shape[0]),
               _strides(query, 4), _strides(key, 4), _strides(cos, 3), _strides(sin, 3), _stream(query))
@@ -271,7 +286,7 @@ def _softmax_cuda(input):
     x = input.contiguous()
     output = torch.empty_like(x)
     width = int(x.shape[-1])
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _call("flux_softmax_f32", x.data_ptr(), output.data_ptr(), x.numel() // width, width, _stream(x))
     return output
 
@@ -300,7 +315,7 @@ def _attention_score_softmax_cuda(scores, additive_attention_mask, scale):
     _check(all(s >= 0 for s in mask.stride()), "flux::attention_score_softmax: negative mask strides are unsupported")
     s = scores.contiguous()
     output = torch.empty_like(s)
-    with torch.cuda.device(s.device):
+    with _on(s.device):
         _call("flux_attention_score_softmax_f32", s.data_ptr(), mask.data_ptr(), output.data_ptr(), float(scale),
               *(int(d) for d in s.shape), _native.length_array([int(d) for d in mask.shape]), _strides(mask, 4),
               _stream(s))
@@ -327,7 +342,7 @@ def _packed_swiglu_shape(packed) -> list:
 
 def _launch_packed_swiglu(packed, output) -> None:
     inter = int(packed.shape[-1]) // 2
-    with torch.cuda.device(packed.device):
+    with _on(packed.device):
         _call("flux_packed_swiglu_f32", packed.data_ptr(), output.data_ptr(), packed.numel() // (2 * inter), inter,
               _stream(packed))
 
@@ -390,7 +405,7 @@ def _launch_gqa(op, query, key_cache, value_cache, mask, scale, cache_length, ou
     tensors = [query, key_cache, value_cache] + ([mask] if mask is not None else [])
     _check(all(s >= 0 for t in tensors for s in t.stride()), f"{op}: negative tensor strides are unsupported")
     _check(key_cache.shape[2] <= _MAX_CAPACITY, f"{op}: cache capacity exceeds {_MAX_CAPACITY} tokens")
-    with torch.cuda.device(query.device):
+    with _on(query.device):
         _call("flux_gqa_decode_attention_strided_f32", query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(),
               _native.ptr(mask), _native.ptr(cache_length), output.data_ptr(), _native.ptr(workspace),
               int(workspace_bytes), float(scale), int(query.shape[1]), int(key_cache.shape[1]),
@@ -480,7 +495,7 @@ def _validate_packed_qkv(packed_qkv, cos, sin, key_cache, value_cache, cache_len
 
 
 def _launch_packed_qkv(packed_qkv, cos, sin, key_cache, value_cache, cache_length, query_output) -> None:
-    with torch.cuda.device(packed_qkv.device):
+    with _on(packed_qkv.device):
         _call("flux_packed_qkv_rope_cache_f32", packed_qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(),
               key_cache.data_ptr(), value_cache.data_ptr(), cache_length.data_ptr(), cache_length.data_ptr(),
               query_output.data_ptr(), int(key_cache.shape[2]), int(packed_qkv.stride(2)), int(cos.stride(2)),
@@ -536,7 +551,7 @@ def _gate_up_out_cuda(input, weight, output):
     op = "flux::packed_gate_up_gemv_out"
     _require_gpu(op, input)
     _check(not _aliases(output, input) and not _aliases(output, weight), f"{op}: output must not alias an input")
-    with torch.cuda.device(input.device):
+    with _on(input.device):
         _call("flux_gate_up_swiglu_f32", input.data_ptr(), None, 0.0, weight.data_ptr(), output.data_ptr(),
               _stream(input))
     return output
@@ -876,7 +891,7 @@ def decode_projection_out(input: torch.Tensor, weight: torch.Tensor, output: tor
            f"{op}: output must be contiguous [1, 1, N]")
     _check(all(t.dtype == torch.float32 for t in (input, weight, output)), f"{op}: tensors must be float32")
     _grad_free(op, input, weight)
-    with torch.cuda.device(input.device):
+    with _on(input.device):
         _call("flux_linear576_f32", input.data_ptr(), weight.data_ptr(), None, output.data_ptr(),
               int(weight.shape[0]), _stream(input))
     return output
