@@ -17,7 +17,7 @@
 // Per layer the phases are
 //   A  norm(h) -> packed QKV GEMV -> RoPE(q,k) -> K/V cache write   (480 waves)
 //   B  split-K GQA attention partials, one (KV head, position chunk) per WG
-//      (one chunk up to 128 attended positions, then one per 64, at most 85 per KV head)
+//      (one chunk up to 224 attended positions, then one per 64, at most 85 per KV head)
 //   B2 merge partials per query head (36 WGs: query head x 16 dims; not with one chunk)
 //   C  o_proj GEMV + residual                                        (576 waves)
 //   D  norm(r) -> packed gate/up GEMV -> SwiGLU                      (1536 waves)
@@ -33,6 +33,7 @@
 #include <cfloat>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 
 namespace flux {
 namespace {
@@ -49,8 +50,8 @@ __device__ __forceinline__ unsigned tid_opaque() {
 
 constexpr int kThreads = 512;
 constexpr int kWavesPerWG = kThreads / kWave;
-constexpr int kAttnRows = 224;            // attention rows per workgroup (LDS-resident K/V)
-constexpr int kSingleChunkRows = 128;     // attended positions that one workgroup per KV head takes whole
+constexpr int kAttnRows = 224;            // attention rows per workgroup (LDS-resident K/V), and the
+                                          // attended positions that one per KV head takes whole
 constexpr int kLmBatch = 4;
 // A wait that has lasted this long (or its bound, if shorter) starts watching the
 // device error word (so one workgroup's timeout ends every other workgroup's wait at
@@ -612,32 +613,27 @@ struct PartialPlainOut {
         }
     }
 };
-// The partial's LL words, or, when one chunk holds every position, the finished head in every copy
-// of the merged vector.
 struct PartialLLOut {
-    uint64_t* ll;  // the layer's parity block
-    int group;
-    int chunk;
-    int chunks;
+    uint64_t* p;
     uint32_t epoch;
     __device__ __forceinline__ void put(int h, int lane, float o, float m, float l) const {
-        // Read through an empty asm, so that nothing derived from it is held across the attention
-        // (0.3% per token at long contexts).
-        int single = chunks;
-        asm volatile("" : "+s"(single));
-        if (single == 1) {
-            const float v = o / l;
-            uint64_t* merged = ll + LLLayout::kAttnMerged + (group * kGroup + h) * kHeadDim + lane;
-#pragma unroll
-            for (int r = 0; r < LLLayout::kReplicas; ++r) ll_store(merged + r * LLLayout::kReplicaStride, v, epoch);
-            return;
-        }
-        uint64_t* slot = ll + LLLayout::kPartials + ((group * chunks + chunk) * kGroup + h) * (kHeadDim + 2);
+        uint64_t* slot = p + h * (kHeadDim + 2);
         ll_store(slot + lane, o, epoch);
         if (lane == 0) {
             ll_store(slot + kHeadDim, m, epoch);
             ll_store(slot + kHeadDim + 1, l, epoch);
         }
+    }
+};
+// A chunk that holds every position: the finished heads, in every copy of the merged vector.
+struct MergedLLOut {
+    uint64_t* p;
+    uint32_t epoch;
+    __device__ __forceinline__ void put(int h, int lane, float o, float m, float l) const {
+        const float v = o / l;
+#pragma unroll
+        for (int r = 0; r < LLLayout::kReplicas; ++r)
+            ll_store(p + r * LLLayout::kReplicaStride + h * kHeadDim + lane, v, epoch);
     }
 };
 
@@ -943,16 +939,18 @@ __global__ void __launch_bounds__(kThreads, 1) fused_decode_kernel(DecodeArgs ar
         // `chunks` (85 on 256 CUs, reached from 5377 positions on).  Short contexts then
         // merge a few partials instead of 85 mostly one-row ones (ctx 128: 0.457 -> 0.427 ms
         // per token, 1024: 0.472 -> 0.436; 64-row chunks measured faster than 32, 96 or 128).
-        // Up to kSingleChunkRows positions one workgroup per KV head takes them all and publishes
-        // the finished heads itself: no merge, no exchange of partials.  Its body takes as long as
-        // a 64-row chunk's (one pass of 128 rows); a second pass and the longer copy would cost
-        // what the merge does.  Per token: 8 positions 377 -> 329 us, 90: 386 -> 356, 128: 388 ->
-        // 375; at 160 positions it measured even, at 190 5% slower.
-        const int want_chunks = attended <= kSingleChunkRows ? 1 : static_cast<int>((attended + 63) >> 6);
+        // Up to kAttnRows positions, one workgroup per KV head takes them all and publishes the
+        // finished heads itself: no merge, no exchange of partials.  It is given no QKV unit, so its
+        // K/V rows are requested before the query exists.  Per token: 8 positions 377 -> 323 us, 90:
+        // 387 -> 333, 128-160: 387 -> 347, 160-192: 393 -> 355.
+        const int want_chunks = attended <= kAttnRows ? 1 : static_cast<int>((attended + 63) >> 6);
         const int tchunks_token = __builtin_amdgcn_readfirstlane(want_chunks < chunks ? want_chunks : chunks);
         const float* emb_row = args.embedding + (token_ok ? token : 0) * kHidden;
 
-        for (int layer = 0; layer < n_layers; ++layer) {
+        // One layer.  Two instances: contexts of one chunk per KV head skip the merge and share the
+        // QKV units differently, and branches for that in one body cost long contexts 1-2%.
+        auto run_layer = [&](const int layer, auto one_chunk_c) __attribute__((always_inline)) {
+            constexpr bool one_chunk = decltype(one_chunk_c)::value;
             int tchunks = tchunks_token;
             asm volatile("" : "+s"(tchunks));
             const LayerWeights Lw = uniform_desc(layer_desc[layer]);
@@ -963,16 +961,21 @@ __global__ void __launch_bounds__(kThreads, 1) fused_decode_kernel(DecodeArgs ar
             float* value_layer = args.value_cache + layer * layer_stride;
 
             // ---- A: norm(h) -> QKV GEMV -> RoPE -> cache (unit = row pair, one per wave) ----
+            // With one chunk per KV head, the last kKVHeads workgroups attend and take no QKV unit:
+            // they need neither h nor an exchange to request their K/V rows, so those are on the
+            // way while the others compute QKV.
+            const bool attends_whole = one_chunk && wg >= G - kKVHeads;
             {
                 FLUX_TRACE_POINT(0);
-                const bool active = gw < kQKV / 2;
+                const int unit = one_chunk ? wave * (G - kKVHeads) + wg : gw;
+                const bool active = unit < kQKV / 2 && !attends_whole;
                 QkvUnitWeights w;
                 float wn[9];
                 RopePair rp{};
                 if (active) {
-                    qkv_load<true>(Lw.qkv, gw, lane, w);
+                    qkv_load<true>(Lw.qkv, unit, lane, w);
                     load_slice576(Lw.input_norm, lane, wn);
-                    rp = rope_pair(cos_row, sin_row, gw);
+                    rp = rope_pair(cos_row, sin_row, unit);
                 }
                 if (layer == 0 && args.hidden_in != nullptr) {
                     // Single-layer step: the caller's hidden state (workgroup 0 also keeps a copy
@@ -984,7 +987,7 @@ __global__ void __launch_bounds__(kThreads, 1) fused_decode_kernel(DecodeArgs ar
                     }
                 } else if (layer == 0) {
                     for (int k = tid_opaque(); k < kHidden; k += kThreads) hvec[k] = token_ok ? emb_row[k] : 0.0f;
-                } else {
+                } else if (!attends_whole) {
                     wg_ll_fetch<2>(ll_prev + replica + LLLayout::kHidden, kHidden, Contiguous{}, epoch_of(counter, layer - 1),
                                    wctx, hvec);
                 }
@@ -993,7 +996,7 @@ __global__ void __launch_bounds__(kThreads, 1) fused_decode_kernel(DecodeArgs ar
                 if (active) {
                     float h[9];
                     lds_slice576(hvec, lane, h);
-                    qkv_unit_compute(w, h, wn, Lw.eps, gw, lane, rp, key_layer + position * kHeadDim,
+                    qkv_unit_compute(w, h, wn, Lw.eps, unit, lane, rp, key_layer + position * kHeadDim,
                                      value_layer + position * kHeadDim, head_stride, QkvLLOut{ll + LLLayout::kQkv, ep});
                 }
             }
@@ -1011,9 +1014,9 @@ __global__ void __launch_bounds__(kThreads, 1) fused_decode_kernel(DecodeArgs ar
 
             // ---- B: attention partial of (KV group g, position chunk c) ----
             FLUX_TRACE_POINT(2);
-            if (wg < kKVHeads * tchunks) {
-                const int g = wg % kKVHeads;
-                const int c = wg / kKVHeads;
+            if (one_chunk ? attends_whole : wg < kKVHeads * tchunks) {
+                const int g = one_chunk ? wg - (G - kKVHeads) : wg % kKVHeads;
+                const int c = one_chunk ? 0 : wg / kKVHeads;
                 int begin32, end32;
                 chunk_range32(static_cast<int>(attended), tchunks, c, begin32, end32);
                 const int64_t begin = begin32, end = end32;
@@ -1054,13 +1057,20 @@ __global__ void __launch_bounds__(kThreads, 1) fused_decode_kernel(DecodeArgs ar
                 FLUX_TRACE_POINT(3);
                 attn_compute(k_lds, v_lds, vec, static_cast<int>(end - begin), Lw.scale * kLog2e,
                              AttnScratch{attn_sp, attn_pl, red},
-                             PartialLLOut{ll, g, c, tchunks, ep}
+                             std::conditional_t<one_chunk, MergedLLOut, PartialLLOut>{
+                                 one_chunk ? ll + LLLayout::kAttnMerged + g * kGroup * kHeadDim
+                                           : ll + LLLayout::kPartials + (g * tchunks + c) * partial_stride,
+                                 ep}
                                  FLUX_TRACE_ARG);
+                // h, the residual of this workgroup's o_proj rows, was not needed before.
+                if (one_chunk && layer > 0)
+                    wg_ll_fetch<2>(ll_prev + replica + LLLayout::kHidden, kHidden, Contiguous{},
+                                   epoch_of(counter, layer - 1), wctx, hvec);
             }
 
             FLUX_TRACE_POINT(4);
             // ---- B2: merge chunk partials; WG (h, quarter) handles 16 dims of query head h ----
-            if (wg < kQHeads * 4 && tchunks != 1) {
+            if (!one_chunk && wg < kQHeads * 4) {
                 const int h = wg >> 2;
                 const int quarter = wg & 3;
                 const int g = h / kGroup;
@@ -1193,6 +1203,11 @@ __global__ void __launch_bounds__(kThreads, 1) fused_decode_kernel(DecodeArgs ar
                 }
                 __syncthreads();
             }
+        };
+        if (tchunks_token == 1) {
+            for (int layer = 0; layer < n_layers; ++layer) run_layer(layer, std::true_type{});
+        } else {
+            for (int layer = 0; layer < n_layers; ++layer) run_layer(layer, std::false_type{});
         }
 
         if (args.hidden_out != nullptr) {

@@ -598,12 +598,13 @@ def test_wait_timeout_reports_error_and_invalid_tokens(small_model):
 
 
 def test_decode_across_the_single_chunk_limit(small_model):
-    """Teacher-forced decode from 126 to 131 attended positions and at 2: up to 128 one workgroup per
-    KV head attends all of them and publishes the finished heads, beyond that two or more chunks are
-    merged.  Each step's logits equal the native prefill's of the extended prompt."""
+    """Teacher-forced decode at 2 attended positions, from 127 to 130 (one pass of the attention's
+    rows, then two) and from 222 to 227: up to 224 one workgroup per KV head attends all positions
+    and publishes the finished heads, beyond that four chunks are merged.  Each step's logits equal
+    the native prefill's of the extended prompt."""
     g = torch.Generator().manual_seed(128)
-    tokens = torch.randint(0, 128, (1, 131), generator=g).cuda()
-    for n_prompt, steps in ((1, 1), (125, 6)):
+    tokens = torch.randint(0, 128, (1, 227), generator=g).cuda()
+    for n_prompt, steps in ((1, 1), (126, 4), (221, 6)):
         runtime = NativeSmolLM2Prefill.capture(small_model, tokens[:, :n_prompt], max_decode_steps=steps)
         for step in range(steps):
             decoded = runtime.replay(tokens[:, n_prompt + step:n_prompt + step + 1])[0, 0].float().cpu().clone()
