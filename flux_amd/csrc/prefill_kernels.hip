@@ -354,22 +354,18 @@ __device__ __forceinline__ void reg_pipeline(Issue&& issue, Compute&& compute) {
     });
 }
 
-template <GemmEpilogue E, int RT, int kCols, bool kNorm, int kK, bool kSumA = false>
+template <GemmEpilogue E, int RT, int kCols, bool kNorm, int kK>
 __global__ void __launch_bounds__(64 * kRegWaves) gemm_reg_kernel(GemmArgs args) {
     static_assert(kK % (kRegWaves * 16) == 0, "whole 16-value stages per wave");
-    static_assert(kCols == 32 || kCols == 64, "16-column blocks of a 32- or 64-column tile");
-    static_assert(kCols == 64 || (E == GemmEpilogue::kStore || E == GemmEpilogue::kResidual),
-                  "column pairs (RoPE, SwiGLU) need 64-column tiles");
+    constexpr bool kPair = E == GemmEpilogue::kQkvRope || E == GemmEpilogue::kSwiglu;
+    static_assert(kCols == 32 || kCols == 64 || (kCols == 16 && !kPair), "16-column blocks, column pairs in two of them");
     static_assert(!kNorm || kK == kHidden, "the folded norm spans the hidden width");
-    static_assert(!kSumA || kSplitBlocksK == 3, "A summed from three planes");
-    constexpr int kAParts = kSumA ? 4 : 1;  // residual + three planes, or the A rows
     constexpr int kJB = kCols / 16;
     constexpr int kRows = 16 * RT;
     constexpr int kStages = kK / (kRegWaves * 16);
-    constexpr int kPerStage = RT * kAParts + kJB + (kNorm ? 1 : 0);  // float4 loads per lane per stage
-    // Ring stages: as many as 72 registers hold (three waves share a SIMD's 512 per lane), 108
-    // when A comes as four parts, so the whole slice is still in flight at once.
-    constexpr int kRingRegs = kSumA ? 108 : 72;
+    constexpr int kPerStage = RT + kJB + (kNorm ? 1 : 0);  // float4 loads per lane per stage
+    // Ring stages: as many as 72 registers hold (three waves share a SIMD's 512 per lane).
+    constexpr int kRingRegs = 72;
     constexpr int kDepthFit = kRingRegs / (4 * kPerStage) < 2 ? 2 : kRingRegs / (4 * kPerStage);
     constexpr int kDepth = kDepthFit < 9 ? kDepthFit : 9;
     __shared__ float partial[kRegWaves][kRows][kCols + 1];
@@ -378,43 +374,35 @@ __global__ void __launch_bounds__(64 * kRegWaves) gemm_reg_kernel(GemmArgs args)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int64_t m0 = static_cast<int64_t>(blockIdx.y) * kRows;
-    const int n0 = static_cast<int>(blockIdx.x) * kCols;
+    // A 32-column tile of a pair epilogue is half of a 64-column group: 16 columns and the 16 that
+    // they pair with, 32 further on.
+    constexpr bool kHalfGroup = kPair && kCols == 32;
+    const int n0 = static_cast<int>(kHalfGroup ? (blockIdx.x >> 1) * 64 : blockIdx.x * kCols);
+    const int sub = kHalfGroup ? 16 * static_cast<int>(blockIdx.x & 1) : 0;
     const int kq = lane >> 4;
     const int r16 = lane & 15;
     const int k_first = wave * (kK / kRegWaves) + 4 * kq;  // this lane's first K value
 
-    // Part 0 is the A rows (or the residual when A is summed); parts 1-3 the planes.
-    const float* a_src[RT][kAParts];
-    int64_t a_row[RT];
+    const float* a_src[RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-        a_row[rt] = m0 + 16 * rt + r16;
-        const int64_t row = a_row[rt] < args.m ? a_row[rt] : args.m - 1;
-        if constexpr (kSumA) {
-            a_src[rt][0] = args.a_residual + row * kK + k_first;
-#pragma unroll
-            for (int b = 0; b < 3; ++b) a_src[rt][1 + b] = args.a_planes + (b * args.m + row) * kK + k_first;
-        } else {
-            a_src[rt][0] = args.a + row * kK + k_first;
-        }
+        const int64_t row = m0 + 16 * rt + r16;
+        a_src[rt] = args.a + (row < args.m ? row : args.m - 1) * kK + k_first;
     }
     const float* b_src[kJB];
 #pragma unroll
     for (int jb = 0; jb < kJB; ++jb)
-        b_src[jb] = args.b + static_cast<int64_t>(b_row<E>(n0 + 16 * jb + r16, args.n)) * kK + k_first;
+        b_src[jb] = args.b + static_cast<int64_t>(b_row<E>(n0 + sub + (kHalfGroup ? 32 : 16) * jb + r16, args.n)) * kK + k_first;
     const float* g_src = kNorm ? args.norm_weight + k_first : nullptr;
 
-    f32x4 ring_a[kDepth][RT][kAParts];
+    f32x4 ring_a[kDepth][RT];
     f32x4 ring_b[kDepth][kJB];
     f32x4 ring_g[kNorm ? kDepth : 1];
     auto issue = [&](auto st) {
         constexpr int s = decltype(st)::value;
         constexpr int slot = s % kDepth;
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int part = 0; part < kAParts; ++part)
-                ring_a[slot][rt][part] = *reinterpret_cast<const f32x4*>(a_src[rt][part] + 16 * s);
+        for (int rt = 0; rt < RT; ++rt) ring_a[slot][rt] = *reinterpret_cast<const f32x4*>(a_src[rt] + 16 * s);
 #pragma unroll
         for (int jb = 0; jb < kJB; ++jb) ring_b[slot][jb] = *reinterpret_cast<const f32x4*>(b_src[jb] + 16 * s);
         if constexpr (kNorm) ring_g[slot] = *reinterpret_cast<const f32x4*>(g_src + 16 * s);
@@ -432,16 +420,7 @@ __global__ void __launch_bounds__(64 * kRegWaves) gemm_reg_kernel(GemmArgs args)
         f32x4 a[RT];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            if constexpr (kSumA) {
-                const f32x4* part = ring_a[slot][rt];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) a[rt][e] = part[0][e] + ((part[1][e] + part[2][e]) + part[3][e]);
-                if (blockIdx.x == 0 && a_row[rt] < args.m)
-                    *reinterpret_cast<f32x4*>(args.a_rows_out + a_row[rt] * kK + k_first + 16 * decltype(st)::value) =
-                        a[rt];
-            } else {
-                a[rt] = ring_a[slot][rt][0];
-            }
+            a[rt] = ring_a[slot][rt];
             if constexpr (kNorm) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -502,12 +481,13 @@ __global__ void __launch_bounds__(64 * kRegWaves) gemm_reg_kernel(GemmArgs args)
         }
     } else {
         // Column pairs j / j + 32 of the 64-column group (the RoPE pair, or gate and up).
-        for (int i = static_cast<int>(threadIdx.x); i < kRows * 32; i += 64 * kRegWaves) {
-            const int row = i / 32, j = i % 32;
+        constexpr int kPairs = kCols / 2;
+        for (int i = static_cast<int>(threadIdx.x); i < kRows * kPairs; i += 64 * kRegWaves) {
+            const int row = i / kPairs, j = i % kPairs;
             const int64_t out_row = m0 + row;
             if (out_row >= args.m) continue;
             const float inv = inv_rms(row);
-            gemm_store_pair<E>(args, out_row, n0, j, total(row, j) * inv, total(row, j + 32) * inv);
+            gemm_store_pair<E>(args, out_row, n0, sub + j, total(row, j) * inv, total(row, j + kPairs) * inv);
         }
     }
 }
@@ -781,21 +761,22 @@ static SplitShape split_shape(const GemmArgs& args, GemmEpilogue epilogue) {
 }
 
 // Tiling of gemm_reg_kernel (rt = 0 when it does not take the GEMM): 16-row blocks with the
-// narrowest column tile whose grid fits the device once (one block per CU), for the GEMMs over
-// the hidden width (QKV, o_proj, gate/up).  The down projection (K = intermediate) measured
-// faster on gemm_split_kernel at every prompt length.
-#ifndef FLUX_REG_GEMM
-#define FLUX_REG_GEMM 1
-#endif
+// narrowest column tile whose grid fits the device once (one block per CU).  For the GEMMs over the
+// hidden width (QKV, o_proj, gate/up) 32 or 64 columns: QKV at 128 rows takes 6.8 us on 32 (half a
+// column group) and 9.1 on 64, gate/up at 20 rows 7.0 and 9.7.  For the down projection
+// (K = intermediate) 16 columns only, i.e. up to 112 rows: 7.1 us against gemm_split_kernel's 8.9
+// (32 columns, or two rounds of 16: 9.9 and 12.2 us at 128 rows).
 struct RegShape {
     int rt;
     int cols;
 };
 static RegShape reg_shape(const GemmArgs& args, GemmEpilogue epilogue) {
-    if (!FLUX_REG_GEMM || args.k != kHidden || args.n % 64 != 0) return {0, 0};
+    if (args.n % 64 != 0) return {0, 0};
     const bool pair = epilogue == GemmEpilogue::kQkvRope || epilogue == GemmEpilogue::kSwiglu;
     const int64_t r16 = (args.m + 15) / 16;
-    if (!pair && (args.n / 32) * r16 <= kSplitBlocks) return {1, 32};
+    if (args.k == kInter && !pair && (args.n / 16) * r16 <= kSplitBlocks) return {1, 16};
+    if (args.k != kHidden) return {0, 0};
+    if ((args.n / 32) * r16 <= kSplitBlocks) return {1, 32};
     if ((args.n / 64) * r16 <= kSplitBlocks) return {1, 64};
     return {0, 0};
 }
@@ -814,21 +795,20 @@ static hipError_t launch_reg(const GemmArgs& args, GemmEpilogue epilogue, RegSha
     const bool norm = args.norm_weight != nullptr;
 #define FLUX_REG(E, COLS, NORM) \
     hipLaunchKernelGGL(HIP_KERNEL_NAME(gemm_reg_kernel<E, 1, COLS, NORM, kHidden>), grid, block, 0, stream, args)
-#define FLUX_REG_PLAIN(E)                       \
-    do {                                        \
-        if (shape.cols == 32) FLUX_REG(E, 32, false); \
-        else FLUX_REG(E, 64, false);            \
+#define FLUX_REG_PLAIN(E)                                                                                            \
+    do {                                                                                                             \
+        if (args.k == kInter)                                                                                        \
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(gemm_reg_kernel<E, 1, 16, false, kInter>), grid, block, 0, stream, args); \
+        else if (shape.cols == 32) FLUX_REG(E, 32, false);                                                           \
+        else FLUX_REG(E, 64, false);                                                                                 \
     } while (0)
-#define FLUX_REG_PAIR(E)                        \
-    do {                                        \
-        if (norm) FLUX_REG(E, 64, true);        \
-        else FLUX_REG(E, 64, false);            \
+#define FLUX_REG_PAIR(E)                                   \
+    do {                                                   \
+        if (shape.cols == 32 && norm) FLUX_REG(E, 32, true); \
+        else if (shape.cols == 32) FLUX_REG(E, 32, false); \
+        else if (norm) FLUX_REG(E, 64, true);              \
+        else FLUX_REG(E, 64, false);                       \
     } while (0)
-    if (args.a_planes != nullptr) {
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(gemm_reg_kernel<GemmEpilogue::kQkvRope, 1, 64, true, kHidden, true>), grid,
-                           block, 0, stream, args);
-        return hipGetLastError();
-    }
     switch (epilogue) {
         case GemmEpilogue::kStore:
             FLUX_REG_PLAIN(GemmEpilogue::kStore);
@@ -878,47 +858,27 @@ static bool split_k_taken(const GemmArgs& args, GemmEpilogue epilogue) {
     return planes_fit(args, kSplitBlocksK) && blocks * kSplitBlocksK <= kSplitKBlocks;
 }
 
-bool gemm_writes_planes(const GemmArgs& args, GemmEpilogue epilogue) {
-    return reg_shape(args, epilogue).rt == 0 && split_k_taken(args, epilogue);
-}
-
-bool gemm_sums_planes(const GemmArgs& args, GemmEpilogue epilogue) {
-    return epilogue == GemmEpilogue::kQkvRope && reg_shape(args, epilogue).rt != 0;
-}
-
 static hipError_t gemm_args_valid(const GemmArgs& args, GemmEpilogue epilogue) {
     if (args.k % kBK != 0 || args.n % 64 != 0 || args.m <= 0) return hipErrorInvalidValue;
     if (epilogue == GemmEpilogue::kSwiglu && args.n % 128 != 0) return hipErrorInvalidValue;
     if (epilogue == GemmEpilogue::kQkvRope && args.n != kQKV) return hipErrorInvalidValue;
     const bool norm = args.norm_weight != nullptr;
     if (norm && !split_folds_norm(args, epilogue)) return hipErrorInvalidValue;
-    if (args.a_planes != nullptr && (!gemm_sums_planes(args, epilogue) || !norm || args.a_residual == nullptr ||
-                                     args.a_rows_out == nullptr || !aligned16(args.a_planes) ||
-                                     !aligned16(args.a_residual) || !aligned16(args.a_rows_out)))
-        return hipErrorInvalidValue;
     return hipSuccess;
 }
 
-static hipError_t launch_gemm_split(const GemmArgs& args, GemmEpilogue epilogue, bool reduce, hipStream_t stream);
+static hipError_t launch_gemm_split(const GemmArgs& args, GemmEpilogue epilogue, hipStream_t stream);
 
 hipError_t launch_gemm(const GemmArgs& args, GemmEpilogue epilogue, hipStream_t stream) {
     const hipError_t valid = gemm_args_valid(args, epilogue);
     if (valid != hipSuccess) return valid;
     const RegShape reg = reg_shape(args, epilogue);
     if (reg.rt != 0) return launch_reg(args, epilogue, reg, stream);
-    return launch_gemm_split(args, epilogue, true, stream);
+    return launch_gemm_split(args, epilogue, stream);
 }
 
-hipError_t launch_gemm_planes(const GemmArgs& args, GemmEpilogue epilogue, hipStream_t stream) {
-    const hipError_t valid = gemm_args_valid(args, epilogue);
-    if (valid != hipSuccess) return valid;
-    if (args.a_planes != nullptr || !gemm_writes_planes(args, epilogue)) return hipErrorInvalidValue;
-    return launch_gemm_split(args, epilogue, false, stream);
-}
-
-// gemm_split_kernel and the remaining kernels of launch_gemm; `reduce` false stops after the
-// partial planes of a K split.
-static hipError_t launch_gemm_split(const GemmArgs& args, GemmEpilogue epilogue, bool reduce, hipStream_t stream) {
+// gemm_split_kernel and the remaining kernels of launch_gemm.
+static hipError_t launch_gemm_split(const GemmArgs& args, GemmEpilogue epilogue, hipStream_t stream) {
     const bool norm = args.norm_weight != nullptr;
     const SplitShape shape = split_shape(args, epilogue);
     const int rt = shape.rt;
@@ -985,7 +945,7 @@ static hipError_t launch_gemm_split(const GemmArgs& args, GemmEpilogue epilogue,
 #undef FLUX_LAUNCH_SPLIT
 #undef FLUX_SPLIT_RT
         hipError_t st = hipGetLastError();
-        if (st != hipSuccess || !split_k || !reduce) return st;
+        if (st != hipSuccess || !split_k) return st;
         const int64_t units = shape.cols == 64 ? args.n / 2 : args.n;
         const dim3 rgrid(static_cast<unsigned>((args.m * units + 255) / 256));
 #define FLUX_REDUCE(E, NORM, COLS) \

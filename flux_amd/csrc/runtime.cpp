@@ -622,12 +622,6 @@ float* PrefillRuntime::prefill(const int64_t* input_ids, hipStream_t stream) {
     return logits_;
 }
 
-// Prompts up to which the down GEMM's partial planes are summed by the next QKV kernel: every
-// one of the QKV kernel's 15 column blocks loads the residual and three planes of its rows, which
-// beyond a few rows costs more than the reduce kernel it replaces (16 tokens: 1.24 against
-// 1.19 ms; 1 token 1.10 → 1.04, 8 tokens 1.16 → 1.13).
-constexpr int64_t kDownPlanesMaxRows = 8;
-
 void PrefillRuntime::run(const int64_t* input_ids, hipStream_t stream) {
     flux_decode_buffers db;
     decode_->buffers(&db);
@@ -645,20 +639,8 @@ void PrefillRuntime::run(const int64_t* input_ids, hipStream_t stream) {
     gu_shape.m = seq_;
     gu_shape.n = kGateUp;
     gu_shape.k = kHidden;
-    GemmArgs down_shape{};
-    down_shape.m = seq_;
-    down_shape.n = kHidden;
-    down_shape.k = kInter;
-    down_shape.split_partials = split_partials_;
-    down_shape.split_floats = split_floats_;
     const bool qkv_folds = gemm_folds_norm(qkv_shape, GemmEpilogue::kQkvRope);
     const bool gu_folds = gemm_folds_norm(gu_shape, GemmEpilogue::kSwiglu);
-    // Prompts of a few tokens: the down GEMM leaves its K-split partial planes unreduced and
-    // the next layer's QKV kernel sums them with the residual into its A rows (writing the
-    // hidden rows on the way), which takes the reduce kernel out of 29 of the 30 layers.
-    const bool down_planes = seq_ <= kDownPlanesMaxRows && qkv_folds &&
-                             gemm_sums_planes(qkv_shape, GemmEpilogue::kQkvRope) &&
-                             gemm_writes_planes(down_shape, GemmEpilogue::kResidual);
     for (int layer = 0; layer < kLayers; ++layer) {
         float* keys = db.key_cache + layer * layer_elems;
         float* values = db.value_cache + layer * layer_elems;
@@ -677,11 +659,6 @@ void PrefillRuntime::run(const int64_t* input_ids, hipStream_t stream) {
         qkv.capacity = capacity_;
         if (layer == 0 || qkv_folds) {
             qkv.a = hidden_a_;
-            if (layer > 0 && down_planes) {
-                qkv.a_planes = split_partials_;  // the previous layer's down GEMM, unreduced
-                qkv.a_residual = hidden_b_;
-                qkv.a_rows_out = hidden_a_;
-            }
             check_hip(launch_norm_gemm(qkv, weights_.input_norm[layer], eps_[layer], norm_, GemmEpilogue::kQkvRope,
                                        stream),
                       "launching input RMSNorm + QKV GEMM");
@@ -734,8 +711,6 @@ void PrefillRuntime::run(const int64_t* input_ids, hipStream_t stream) {
         if (layer + 1 < kLayers && !qkv_folds) {
             check_hip(launch_gemm_residual_norm(dn, weights_.input_norm[layer + 1], eps_[layer + 1], norm_, stream),
                       "launching down GEMM + next input RMSNorm");
-        } else if (layer + 1 < kLayers && down_planes) {
-            check_hip(launch_gemm_planes(dn, GemmEpilogue::kResidual, stream), "launching down GEMM (partial planes)");
         } else {
             check_hip(launch_gemm(dn, GemmEpilogue::kResidual, stream), "launching down GEMM");
         }
