@@ -40,8 +40,8 @@ __device__ __forceinline__ void lds_copy16(const float* src, float* lds) {
 // Grids smaller than the device (short and mid-length prompts): one block per
 // (32 * RT) x 64 output tile, RT = 1, 2 or 4.  Its kSplitWaves waves are RT row tiles
 // of 32 times kSplitWaves / RT contiguous K ranges.  A wave streams its 32 A rows and the
-// tile's 64 B rows over its K range, 16 K values (64 bytes per row) at a time, laid out
-// and swizzled as in gemm_kernel, through a private ring of kSplitStages LDS buffers;
+// tile's 64 B rows over its K range, 16 K values (64 bytes per row) at a time, 16-byte
+// pieces XOR-swizzled by (row >> 2) & 3, through a private ring of kSplitStages LDS buffers;
 // while a stage's MFMAs run, the next stage's operands are already in registers and the
 // kSplitStages - 2 after it are being copied.  No wave waits for another until the
 // partial tiles of one row tile meet in LDS (RT < 4).  They are summed in K order (the
@@ -591,9 +591,8 @@ __global__ void __launch_bounds__(256) split_reduce_residual_norm_kernel(GemmArg
 // and the 9 x (M / 64) blocks are small enough to spread evenly over the CUs.  A
 // stage is 32 K values, one 128-byte line per row (16-byte pieces XOR-swizzled so a
 // 16-lane read pass covers all 64 banks), streamed through a ring of four LDS buffers
-// with three copies in flight, stepped as in gemm_ring_kernel.  For every grid size:
-// at 8192 rows the ring measured 0.3 ms per prefill faster than two buffers (which
-// fit more blocks per CU but wait on each stage's copy).
+// with three copies in flight, counted waits and one barrier per stage (two buffers fit
+// more blocks per CU but wait on each stage's copy, and measured slower).
 template <GemmEpilogue E>
 __global__ void __launch_bounds__(kGemmThreads) gemm_narrow_kernel(GemmArgs args) {
     static_assert(E == GemmEpilogue::kStore || E == GemmEpilogue::kResidual, "plain epilogues only");
