@@ -201,8 +201,28 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_limb_kernel(GemmArgs args) {
         if (s + 1 < stages) stage(odd, s + 1);
     }
 
-    if (__syncthreads_or(!(largest <= kLimbMax))) {
-        // An infinity, or a magnitude bf16 cannot hold: this tile on the float32 instruction.
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
+    // A tile on the float32 instruction: one with an infinity, or a magnitude bf16 cannot hold, and
+    // one with a value that is not finite, since where the leading products overflow to one
+    // infinity the small ones may overflow to the other.
+    float finite[TM][TN];  // zero times every value: zero if they are finite
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            finite[i][j] = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) finite[i][j] = fmaf(acc[i][j][r], 0.0f, finite[i][j]);
+        }
+    bool redo = !(largest <= kLimbMax);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) redo |= finite[i][j] != 0.0f;
+    if (__syncthreads_or(redo)) {
         clear();
 #pragma unroll 1
         for (int k = k_first + 4 * h; k < k_first + span; k += 8) {
@@ -227,10 +247,6 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_limb_kernel(GemmArgs args) {
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
         }
     }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
     const int g0 = n0 + wn * 64;
     if (g0 >= args.n) return;
     if constexpr (kKB > 1) {

@@ -71,6 +71,55 @@ def test_limb_linear_keeps_float32_range(gpu_device):
     torch.testing.assert_close(c[rows].double(), a[rows].double() @ w.double().T, rtol=1e-4, atol=1e-4)
 
 
+def _rows_call(name, x, w, device):
+    """The GEMM `name` on rows `x`, and the same with float64 products."""
+    rows = x.shape[0]
+    if name == "linear":
+        return _linear(x, w, None, device), x.double() @ w.double().T
+    lib, stream = _native.load(), _native.current_stream(device)
+    exact = x.double() @ w.double().T
+    x, w = x.to(device), w.to(device)
+    if name == "gate_up":
+        out = torch.empty(rows, 1536, device=device)
+        _native.check(lib.flux_gate_up_swiglu_rows_f32(x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, stream))
+        gate, up = exact.chunk(2, dim=-1)
+        want = gate / (1 + torch.exp(-gate)) * up
+    else:
+        # cos = 1, sin = 0: the rotation adds 0 times the paired column.
+        cos, sin = torch.ones(rows, 64, device=device), torch.zeros(rows, 64, device=device)
+        out = torch.empty(15, rows, 64, device=device)
+        _native.check(lib.flux_qkv_rope_cache_rows_f32(x.data_ptr(), w.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+                                                       rows, out[:9].data_ptr(), out[9:12].data_ptr(),
+                                                       out[12:].data_ptr(), rows, stream))
+        heads = exact.view(rows, 15, 64).transpose(0, 1)
+        paired = torch.cat((-heads[:12, :, 32:], heads[:12, :, :32]), dim=-1)
+        want = torch.cat((heads[:12] + paired.float() * 0.0, heads[12:]))
+    torch.cuda.synchronize()
+    return out.cpu(), want
+
+
+# 2500 rows: the limb kernel under each epilogue.
+@pytest.mark.parametrize("name,n", [("linear", 576), ("gate_up", 3072), ("qkv", 960)])
+def test_limb_gemm_overflow_is_infinite(gpu_device, name, n):
+    # Products of finite values that overflow: the leading limbs' to one infinity, of a small pair
+    # of limbs possibly to the other.
+    x, w = _randn(2500, 576, seed=30), _randn(n, 576, seed=31, std=0.05)
+    if name == "gate_up":
+        w[:1536, [7, 11]] = 0.0  # the gates stay ordinary
+    up = n - 100  # a column of up, of a value head, or any
+    x[3, 7], w[up, 7] = 1.3e25, 1.7e25
+    x[2499, 11], w[up + 1, 11] = 1.234e22, -5.678e22
+    got, want = _rows_call(name, x, w, gpu_device)
+    want = want.float()
+    assert int(torch.isinf(want).sum()) == 2
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+    ordinary = [r for r in range(2500) if r not in (3, 2499)]
+    got, want = ((t.movedim(-2, 0)[ordinary]).flatten(1) for t in (got, want))
+    columns = [c for c in range(want.shape[1]) if c not in (up % want.shape[1], up % want.shape[1] + 1)]
+    torch.testing.assert_close(got[:, columns], want[:, columns], rtol=5e-4, atol=1e-4)
+
+
 def _attention(q, k, v, device):
     lib = _native.load()
     seq = q.shape[1]
