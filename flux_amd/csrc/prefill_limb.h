@@ -10,9 +10,10 @@
 // K = 1536: 6.0e-7 against 6.8e-7).  Six of these instructions take 192 cycles for sixteen K
 // values, eight of the float32 ones 512.
 //
-// Limbs cannot carry infinities (inf - inf), nor magnitudes above the largest bf16: kernels
-// track the largest magnitude they split and take the float32 instruction when it is above
-// kLimbMax.  NaN propagates through the limbs by itself.
+// That holds from 2^-110 to the largest bf16.  Limbs cannot carry infinities (inf - inf) nor
+// magnitudes above (kLimbMax), bf16 has no bits below 2^-133 for the low limbs of smaller values
+// (kLimbMin), and overflowing limb products need not agree in sign: kernels find out whether any
+// of these shows in what they computed, and then compute it with the float32 instruction.
 #pragma once
 
 #include "prefill_common.h"
@@ -29,6 +30,7 @@ typedef f32x4 f32x4_u __attribute__((aligned(4)));
 
 constexpr int kLimbs = 3;
 constexpr float kLimbMax = 3.3895313892515355e38f;  // largest finite bf16 (0x7f7f)
+constexpr float kLimbMin = 0x1p-110f;               // and the least magnitude whose limbs add up to it
 
 // The limbs of eight values, as MFMA operands.
 struct Limbs8 {
@@ -69,6 +71,9 @@ __device__ __forceinline__ Limbs8 split8(const f32x4& lo, const f32x4& hi) {
 __device__ __forceinline__ void track_max(float& running, float a, float b) {
     asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(running) : "v"(a), "v"(b));
 }
+
+// Whether the limbs of a value may not add up to it (they are then within 2^-134 of it).
+__device__ __forceinline__ bool limbs_drop(float v) { return v != 0.0f && fabsf(v) < kLimbMin; }
 
 __device__ __forceinline__ f32x16 mfma_bf16(const u32x4& a, const u32x4& b, const f32x16& c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,

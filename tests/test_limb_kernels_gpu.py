@@ -71,6 +71,10 @@ def test_limb_linear_keeps_float32_range(gpu_device):
     torch.testing.assert_close(c[rows].double(), a[rows].double() @ w.double().T, rtol=1e-4, atol=1e-4)
 
 
+def _rel(got, want):
+    return float((got - want).norm() / want.norm())
+
+
 def _rows_call(name, x, w, device):
     """The GEMM `name` on rows `x`, and the same with float64 products."""
     rows = x.shape[0]
@@ -118,6 +122,26 @@ def test_limb_gemm_overflow_is_infinite(gpu_device, name, n):
     got, want = ((t.movedim(-2, 0)[ordinary]).flatten(1) for t in (got, want))
     columns = [c for c in range(want.shape[1]) if c not in (up % want.shape[1], up % want.shape[1] + 1)]
     torch.testing.assert_close(got[:, columns], want[:, columns], rtol=5e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("small", [2.0 ** -120, 1e-38, 1e-41])
+@pytest.mark.parametrize("of", ["x", "w"])
+@pytest.mark.parametrize("name,n", [("linear", 576), ("gate_up", 3072), ("qkv", 960)])
+def test_limb_gemm_small_magnitudes(gpu_device, name, n, of, small):
+    # Rows, or weights, of which bf16 limbs keep only the leading bits or none: as close as others
+    # (the float32 instruction is at 4.4e-7 for K = 576; SwiGLU multiplies two such sums).
+    x, w = _randn(2500, 576, seed=32), _randn(n, 576, seed=33, std=0.05)
+    if of == "x":
+        x[1200:1300] *= small
+        w *= 2.0 ** 100
+    else:
+        w *= small
+        x *= 2.0 ** 100
+    got, want = _rows_call(name, x, w, gpu_device)
+    if of == "x":
+        rows = (lambda t: t[:, 1200:1300]) if name == "qkv" else (lambda t: t[1200:1300])
+        got, want = rows(got), rows(want)
+    assert _rel(got.double(), want) < 1e-6
 
 
 def _attention(q, k, v, device):
