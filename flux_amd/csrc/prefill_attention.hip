@@ -398,14 +398,18 @@ prefill_attention_f32_kernel(const float* __restrict__ q, const float* __restric
 // [key half][step][dim half][limb][lane half][32 dims] x 8 values, whose slot e holds key
 // 8 (2 step + e / 4) + 4 (lane half) + e % 4 of the half: the keys whose probabilities a lane
 // holds after S^T.  Block (KV head, tile); rows past the prompt repeat its last row (masked).
-// flags[block] tells that a value of the tile is infinite or above the largest bf16.
+// flags[block] tells that a key of the tile is above kLimbMaxScore or a value above kLimbMaxValue.
 constexpr int kLimbTile = kKTile * kHeadDim * 2 * kLimbs;  // bytes of one K or V tile: 24576
+// Magnitudes up to which no sum of products overflows (64 of a scaled query and a key, at most 2048
+// of a weight and a value), which those of small limbs could do to another sign than the whole.
+constexpr float kLimbMaxScore = 0x1p60f;
+constexpr float kLimbMaxValue = 0x1p100f;
 
-__device__ __forceinline__ bool too_large(const float (&v)[8]) {
+__device__ __forceinline__ bool above(const float (&v)[8], float most) {
     float m = 0.0f;
 #pragma unroll
     for (int e = 0; e < 8; e += 2) track_max(m, v[e], v[e + 1]);
-    return !(m <= kLimbMax);
+    return !(m <= most);
 }
 
 __device__ __forceinline__ void store_limbs(char* at, const float (&v)[8]) {
@@ -434,7 +438,7 @@ __global__ void __launch_bounds__(256) attention_limbs_kernel(const float* __res
         const int64_t row = key0 + key < seq ? key0 + key : seq - 1;
         *reinterpret_cast<f32x4*>(v) = *reinterpret_cast<const f32x4*>(kg + row * kHeadDim + 8 * part);
         *reinterpret_cast<f32x4*>(v + 4) = *reinterpret_cast<const f32x4*>(kg + row * kHeadDim + 8 * part + 4);
-        large |= too_large(v);
+        large |= above(v, kLimbMaxScore);
         store_limbs(kp + ((key >> 5) * 4 + (part >> 1)) * 3072 + (part & 1) * 512 + (key & 31) * 16, v);
     }
 #pragma unroll
@@ -447,7 +451,7 @@ __global__ void __launch_bounds__(256) attention_limbs_kernel(const float* __res
             const int64_t key = key0 + 16 * step + 8 * (e >> 2) + 4 * half + (e & 3);
             v[e] = vg[(key < seq ? key : seq - 1) * kHeadDim + dim];
         }
-        large |= too_large(v);
+        large |= above(v, kLimbMaxValue);
         store_limbs(vp + (step * 2 + (dim >> 5)) * 3072 + half * 512 + (dim & 31) * 16, v);
     }
     const int any = __syncthreads_or(large);
@@ -491,7 +495,7 @@ prefill_attention_kernel(const float* __restrict__ q, const float* __restrict__ 
             const f32x4 lo = *reinterpret_cast<const f32x4*>(qp + 16 * t) * s2;
             const f32x4 hi = *reinterpret_cast<const f32x4*>(qp + 16 * t + 4) * s2;
             const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            large |= too_large(v);
+            large |= above(v, kLimbMaxScore);
             const Limbs8 l = split8(lo, hi);
 #pragma unroll
             for (int j = 0; j < kLimbs; ++j) qreg[t][j] = l.limb[j];

@@ -202,3 +202,15 @@ def test_limb_attention_keeps_float32_range(gpu_device):
     assert torch.all(got[6:, 1000:, 5] == float("inf"))
     rest = [d for d in range(64) if d != 5]
     torch.testing.assert_close(got[6:, :, rest], want[6:, :, rest], rtol=2e-4, atol=2e-5)
+
+
+def test_limb_attention_overflow_is_infinite(gpu_device):
+    # Scores whose products overflow to minus infinity, a small pair of limbs' to plus infinity:
+    # queries from 1000 on cannot see key 700.
+    seq = 1500
+    q, k, v = _randn(9, seq, 64, seed=40), _randn(3, seq, 64, seed=41), _randn(3, seq, 64, seed=42)
+    q[:3, :, 0], k[0, :, 0] = 0.0, 0.0
+    q[:3, 1000:, 0], k[0, 700, 0] = 1.3e25, -1.7e25
+    got = _attention(q, k, v, gpu_device)
+    want = _attention64(q, k, v)  # a score of -4e49 has no weight in float64 either
+    torch.testing.assert_close(got, want, rtol=2e-4, atol=2e-5)
