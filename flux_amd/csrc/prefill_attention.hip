@@ -401,9 +401,12 @@ prefill_attention_f32_kernel(const float* __restrict__ q, const float* __restric
 // flags[block] tells that a key of the tile is above kLimbMaxScore or a value above kLimbMaxValue.
 constexpr int kLimbTile = kKTile * kHeadDim * 2 * kLimbs;  // bytes of one K or V tile: 24576
 // Magnitudes up to which no sum of products overflows (64 of a scaled query and a key, at most 2048
-// of a weight and a value), which those of small limbs could do to another sign than the whole.
+// of a weight and a value), which those of small limbs could do to another sign than the whole, and
+// up to which bits that limbs do not carry (at most 2^-134 of each factor, limbs_drop) change a
+// score by less than 2^-66, a weight by as little, and a sum over n key tiles by less than 2^-108 n.
 constexpr float kLimbMaxScore = 0x1p60f;
-constexpr float kLimbMaxValue = 0x1p100f;
+constexpr float kLimbMaxValue = 0x1p19f;
+constexpr float kLimbSureSum = 0x1p-82f;  // per key tile: from here on that is under 2^-26 of a sum
 
 __device__ __forceinline__ bool above(const float (&v)[8], float most) {
     float m = 0.0f;
@@ -458,20 +461,15 @@ __global__ void __launch_bounds__(256) attention_limbs_kernel(const float* __res
     if (threadIdx.x == 0) flags[blockIdx.x] = any;
 }
 
-__global__ void __launch_bounds__(kAttnThreads, 2)
-prefill_attention_kernel(const float* __restrict__ q, const float* __restrict__ key_cache,
-                         const float* __restrict__ value_cache, const char* __restrict__ k_planes,
-                         const char* __restrict__ v_planes, const int* __restrict__ flags, int64_t seq,
-                         int64_t capacity, float scale, float* __restrict__ workspace, float* __restrict__ out_rows) {
-    __shared__ __align__(16) char ks[kLimbTile];
-    __shared__ __align__(16) char v0s[kLimbTile];
-    __shared__ __align__(16) char v1s[kLimbTile];
-
+// One block's item on limb products; false, and nothing written, where it needs the float32
+// instruction.
+__device__ __forceinline__ bool attention_item_limbs(const float* __restrict__ q, const char* __restrict__ k_planes,
+                                                    const char* __restrict__ v_planes, const int* __restrict__ flags,
+                                                    int64_t seq, float scale, float* __restrict__ workspace,
+                                                    float* __restrict__ out_rows, int h, int64_t qt, int64_t chunk,
+                                                    char* ks, char* v0s, char* v1s, int* unsure) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int h = static_cast<int>(blockIdx.x % kQHeads);
-    int64_t qt, chunk;
-    attn_item(seq, blockIdx.x / kQHeads, qt, chunk);
     const int g = h / kGroup;
     const int64_t qw0 = qt * kQTile + 32 * wave;  // first query of this wave
     const int col = lane & 31;
@@ -501,12 +499,8 @@ prefill_attention_kernel(const float* __restrict__ q, const float* __restrict__ 
             for (int j = 0; j < kLimbs; ++j) qreg[t][j] = l.limb[j];
         }
         if (kt_begin + lane < kt_end) large |= flags[g * tiles + kt_begin + lane] != 0;
-        if (__syncthreads_or(large)) {
-            attention_item_f32(q, key_cache, value_cache, seq, capacity, scale, workspace, out_rows, h, qt, chunk,
-                               reinterpret_cast<float*>(ks), reinterpret_cast<float*>(v0s),
-                               reinterpret_cast<float*>(v1s));
-            return;
-        }
+        if (threadIdx.x == 0) *unsure = 0;
+        if (__syncthreads_or(large)) return false;
     }
 
     // Copies of key tile kt: 24 of 1 KB each for K and V, wave w issues w, w + 4, ...
@@ -656,23 +650,37 @@ prefill_attention_kernel(const float* __restrict__ q, const float* __restrict__ 
     issue(vg, v0s, kt_begin);
     __builtin_amdgcn_s_waitcnt(0);
     lds_barrier();
-    for (int64_t kt = kt_begin; kt < kt_end; kt += 2) {
+    for (int64_t kt = kt_begin;; kt += 2) {
         const int64_t n1 = kt + 1 < kt_end ? kt + 1 : kt_end - 1;
         issue(vg, v1s, n1);
         tile(v0s, kt, n1);
+        if (kt + 1 >= kt_end) break;
         __builtin_amdgcn_s_waitcnt(0);  // this wave's copies of tile kt + 1 have landed
         lds_barrier();
-        if (kt + 1 < kt_end) {
-            const int64_t n2 = kt + 2 < kt_end ? kt + 2 : kt_end - 1;
-            issue(vg, v0s, n2);
-            tile(v1s, kt + 1, n2);
-            __builtin_amdgcn_s_waitcnt(0);
-            lds_barrier();
-        }
+        const int64_t n2 = kt + 2 < kt_end ? kt + 2 : kt_end - 1;
+        issue(vg, v0s, n2);
+        tile(v1s, kt + 1, n2);
+        if (kt + 2 >= kt_end) break;
+        __builtin_amdgcn_s_waitcnt(0);
+        lds_barrier();
     }
 
     // O^T accumulator: lane holds dims 32 db + 8 (r / 4) + 4 half + r % 4 of query my_q.
-    if (my_q >= seq) return;
+    // A sum below kLimbSureSum may lack bits: the smallest, exact zeros aside (those are of values
+    // that are zero, or of products that float32 does not hold either).
+    unsigned least = ~0u;
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            o_acc[db][r] += o_low[db][r];
+            least = min(least, magnitude_key(o_acc[db][r]));
+        }
+    if (least < magnitude_key(kLimbSureSum * static_cast<float>(kt_end - kt_begin))) *unsure = 1;
+    __builtin_amdgcn_s_waitcnt(0);  // no copy may still be landing in LDS when the block retires or starts again
+    lds_barrier();
+    if (*unsure != 0) return false;
+    if (my_q >= seq) return true;
     const bool single = attn_chunks(seq, qt) == 1;
     const float inv = single ? 1.0f / l_run : 1.0f;
     float* dst = single ? out_rows + my_q * kHidden + h * kHeadDim
@@ -683,10 +691,29 @@ prefill_attention_kernel(const float* __restrict__ q, const float* __restrict__ 
         for (int r = 0; r < 16; r += 4) {
             f32x4 o;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = (o_acc[db][r + e] + o_low[db][r + e]) * inv;
+            for (int e = 0; e < 4; ++e) o[e] = o_acc[db][r + e] * inv;
             *reinterpret_cast<f32x4*>(dst + 32 * db + 2 * r + 4 * half) = o;
         }
     if (!single && half == 0) *reinterpret_cast<float2*>(dst + kHeadDim) = make_float2(m_run, l_run);  // m in log2 units
+    return true;
+}
+
+__global__ void __launch_bounds__(kAttnThreads, 2)
+prefill_attention_kernel(const float* __restrict__ q, const float* __restrict__ key_cache,
+                         const float* __restrict__ value_cache, const char* __restrict__ k_planes,
+                         const char* __restrict__ v_planes, const int* __restrict__ flags, int64_t seq,
+                         int64_t capacity, float scale, float* __restrict__ workspace, float* __restrict__ out_rows) {
+    __shared__ __align__(16) char ks[kLimbTile];
+    __shared__ __align__(16) char v0s[kLimbTile];
+    __shared__ __align__(16) char v1s[kLimbTile];
+    __shared__ int unsure;  // some sum may lack bits that limbs do not carry
+    const int h = static_cast<int>(blockIdx.x % kQHeads);
+    int64_t qt, chunk;
+    attn_item(seq, blockIdx.x / kQHeads, qt, chunk);
+    if (!attention_item_limbs(q, k_planes, v_planes, flags, seq, scale, workspace, out_rows, h, qt, chunk, ks, v0s,
+                              v1s, &unsure))
+        attention_item_f32(q, key_cache, value_cache, seq, capacity, scale, workspace, out_rows, h, qt, chunk,
+                           reinterpret_cast<float*>(ks), reinterpret_cast<float*>(v0s), reinterpret_cast<float*>(v1s));
 }
 
 // Combines the chunk partials of query tiles with more than one chunk.  Block

@@ -72,6 +72,9 @@ __device__ __forceinline__ void track_max(float& running, float a, float b) {
     asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(running) : "v"(a), "v"(b));
 }
 
+// Orders magnitudes as integers (an addition and a minimum, against two comparisons), zero last.
+__device__ __forceinline__ unsigned magnitude_key(float v) { return 2 * __float_as_uint(v) - 1; }
+
 // Whether the limbs of a value may not add up to it (they are then within 2^-134 of it).
 __device__ __forceinline__ bool limbs_drop(float v) { return v != 0.0f && fabsf(v) < kLimbMin; }
 

@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 import ctypes
+import math
 
 import pytest
 import torch
@@ -214,3 +215,32 @@ def test_limb_attention_overflow_is_infinite(gpu_device):
     got = _attention(q, k, v, gpu_device)
     want = _attention64(q, k, v)  # a score of -4e49 has no weight in float64 either
     torch.testing.assert_close(got, want, rtol=2e-4, atol=2e-5)
+
+
+def test_limb_attention_small_magnitudes(gpu_device):
+    # Keys, queries and values of which bf16 limbs keep only the leading bits, one per KV head; every
+    # output is as close as with ordinary magnitudes.
+    seq = 1100
+    q, k, v = _randn(9, seq, 64, seed=43), _randn(3, seq, 64, seed=44), _randn(3, seq, 64, seed=45)
+    k[0] *= 2.0 ** -120
+    q[:3] *= 2.0 ** 120
+    k[1] *= 2.0 ** 122
+    q[3:6] *= 2.0 ** -122
+    v[2] *= 2.0 ** -121
+    got, want = _attention(q, k, v, gpu_device), _attention64(q, k, v)
+    for g in range(3):
+        assert _rel(got[3 * g:3 * g + 3], want[3 * g:3 * g + 3]) < 1e-6
+
+
+def test_limb_attention_small_weights(gpu_device):
+    # Every query's weight is on the first key, whose values are zero; the outputs are the others',
+    # with weights of about 2^-123.  A score of -123 is known to half a unit in the last place,
+    # 2^-18, and so are these weights to 2.6e-6.
+    seq = 1100
+    q, k, v = _randn(9, seq, 64, seed=46, std=0.1), _randn(3, seq, 64, seed=47), _randn(3, seq, 64, seed=48)
+    q[:, :, 0], k[:, :, 0] = 10.0, 0.0
+    k[:, 0] = 0.0
+    k[:, 0, 0] = 123 * math.log(2) / 1.25
+    v[:, 0] = 0.0
+    got, want = _attention(q, k, v, gpu_device), _attention64(q, k, v)
+    assert _rel(got[:, 64:], want[:, 64:]) < 1e-5
