@@ -736,7 +736,9 @@ constexpr int64_t kSplitKBlocks = 256;  // ... and with K split over blocks whil
 // gemm_narrow_kernel (64 x 64 tiles over all of K) while its grid fits the device once.  It takes
 // what is left then without partial planes, e.g. one layer's o_proj up to 1792 rows: a limb block
 // is longer than one of its blocks there (1000 rows, K = 576: 21 against 13 us; K = 1536, 1536
-// rows: 49 against 31), and shorter beyond (2048 rows: 21 against 25; 49 against 57).
+// rows: 49 against 31; 500 x 1024, K = 64: 6.2 against 4.9, K = 1024: 33 against 20), and shorter
+// beyond (2048 rows: 21 against 25; 49 against 57).  Only below K = 128 is it even with limb
+// tiles on two rounds of blocks.
 constexpr int64_t kNarrowBlocks = 256;
 
 // Tiling of gemm_split_kernel for this GEMM (rt = 0 when it does not take it), for K = 576
@@ -842,8 +844,8 @@ static int limb_max_parts(const GemmArgs& args, GemmEpilogue epilogue) {
 }
 
 static bool narrow_taken(const GemmArgs& args, GemmEpilogue epilogue) {
-    return (epilogue == GemmEpilogue::kStore || epilogue == GemmEpilogue::kResidual) && args.n % 128 != 0 &&
-           args.k % 32 == 0 && static_cast<int64_t>(args.n / 64) * ((args.m + 63) / 64) <= kNarrowBlocks;
+    return (epilogue == GemmEpilogue::kStore || epilogue == GemmEpilogue::kResidual) && args.k % 32 == 0 &&
+           static_cast<int64_t>(args.n / 64) * ((args.m + 63) / 64) <= kNarrowBlocks;
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }

@@ -56,3 +56,13 @@ def test_qkv_rows(gpu_device, rows):
     rotated = heads * cos.double() + turned * sin.double()
     for got, want in ((q, rotated[:9]), (k, rotated[9:12]), (v, heads[12:])):
         torch.testing.assert_close(got.cpu().double(), want, rtol=1e-4, atol=1e-5)
+
+
+# Widths that are multiples of 128: 64 x 64 tiles while at most 256 of them, limb tiles beyond.
+@pytest.mark.parametrize("rows,n,k", [(1, 128, 64), (8192, 128, 64), (8193, 128, 64), (65, 3072, 64), (321, 3072, 96)])
+def test_linear_rows_of_wide_tiles(gpu_device, rows, n, k):
+    a, w, r = _randn(rows, k, seed=10), _randn(n, k, seed=11), _randn(rows, n, seed=12)
+    out = torch.empty(rows, n, device=gpu_device)
+    _call("flux_linear_f32", a.to(gpu_device), w.to(gpu_device), r.to(gpu_device), out, rows, n, k)
+    want = a.double() @ w.double().T + r.double()
+    assert torch.all((out.cpu().double() - want).abs() <= _bound(a, w) + want.abs() * 2.0 ** -23)
