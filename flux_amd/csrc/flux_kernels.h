@@ -121,32 +121,24 @@ struct GemmArgs {
     float* key_cache;       // [3, capacity, 64]
     float* value_cache;
     int64_t capacity;
-    // Optional RMSNorm folded into the GEMM (only gemm_split_kernel takes it): A holds the
-    // raw rows, each K value is scaled by norm_weight[k] and each output row by the inverse
-    // RMS of its A row.  launch_gemm rejects a norm it cannot fold; launch_norm_gemm folds it
-    // where it can and otherwise runs the RMSNorm kernel first.
+    // Optional RMSNorm folded into the GEMM (only gemm_reg_kernel and gemm_split_kernel take it): A
+    // holds the raw rows, each K value is scaled by norm_weight[k] and each output row by the
+    // inverse RMS of its A row.  launch_gemm rejects a norm it cannot fold; launch_norm_gemm folds
+    // it where it can and otherwise runs the RMSNorm kernel first.
     const float* norm_weight;
     float norm_eps;
-    // Optional workspace (split_partials_floats(M, N) floats) that lets launch_gemm split K
-    // over kSplitBlocksK (or, for the 576-column kernel, two) blocks when the grid leaves CUs
-    // idle: one partial plane [M, N] per K part, then kSplitBlocksK partial row sums of
-    // squares [M] (folded norm), summed in order by a second kernel that applies the
-    // epilogue.  Null: every block covers all of K.
+    // Optional workspace (split_partials_floats(M, N) floats) that lets a GEMM with the residual
+    // epilogue split K over two or kSplitBlocksK blocks where that is faster: one partial plane
+    // [M, N] per K part, summed in order by a second kernel that adds the residual.  Null: every
+    // block covers all of K.
     float* split_partials;
     int64_t split_floats;  // floats available at split_partials: no split whose planes exceed it
 };
 
-// Blocks that share one output tile's K range when GemmArgs::split_partials is given.
+// Most blocks that share one output tile's K range when GemmArgs::split_partials is given.
 constexpr int kSplitBlocksK = 3;
-// Prompt lengths up to which the prefill runtime provides the partial planes (longer
-// prompts fill the device without splitting K): for the widest GEMM (gate/up) up to
-// kSplitKMaxRows rows, for the 576-column GEMMs up to kNarrowSplitMaxRows.
-constexpr int64_t kSplitKMaxRows = 1024;
-constexpr int64_t kNarrowSplitMaxRows = 16384;
 // Floats of GemmArgs::split_partials for an [M, N] GEMM.
-__host__ __device__ constexpr int64_t split_partials_floats(int64_t m, int64_t n) {
-    return kSplitBlocksK * m * n + kSplitBlocksK * m;
-}
+__host__ __device__ constexpr int64_t split_partials_floats(int64_t m, int64_t n) { return kSplitBlocksK * m * n; }
 
 // GEMMs on three-limb bf16 products (prefill_limb_kernels.hip): block rows (256, 128 or 64 of
 // 128 columns) and K parts; parts > 1 leave that many partial planes in args.split_partials.

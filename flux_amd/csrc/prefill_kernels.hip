@@ -59,9 +59,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 // kStages = K / (kSplitWaves / RT * 16), fixed at compile time so the stage loop is
 // straight-line code and every wait names exactly the copies it needs.
-// kKB > 1: blockIdx.x = column tile * kKB + kb, and block kb covers the kb-th third of K;
-// instead of the epilogue it writes its summed tile (and its rows' partial sums of squares)
-// to partial plane kb of args.split_partials for gemm_split_reduce_kernel.
+// kKB > 1 (the down projection of 113 to 128 rows): blockIdx.x = column tile * kKB + kb, and block
+// kb covers the kb-th third of K; instead of the epilogue it writes its summed tile to partial
+// plane kb of args.split_partials for split_reduce_residual_kernel.
 template <GemmEpilogue E, int kStages, int RT, bool kNorm, int kCols, int kKB>
 __global__ void __launch_bounds__(64 * kSplitWaves) gemm_split_kernel(GemmArgs args) {
     static_assert(kSplitStages == 5, "the buffers below are spelled out");
@@ -71,6 +71,7 @@ __global__ void __launch_bounds__(64 * kSplitWaves) gemm_split_kernel(GemmArgs a
     static_assert(kCols == 64 || (kCols == 32 && !kNorm &&
                                   (E == GemmEpilogue::kStore || E == GemmEpilogue::kResidual)),
                   "32-column tiles carry no column pairs");
+    static_assert(kKB == 1 || (kCols == 32 && RT == 1), "partial planes of 32-column tiles only");
     constexpr int kTiles = kCols / 32;
     constexpr int kRows = 32 + kCols;  // A rows + B rows per stage
     constexpr int kCopies = kRows / 16;
@@ -233,51 +234,19 @@ __global__ void __launch_bounds__(64 * kSplitWaves) gemm_split_kernel(GemmArgs a
         return rms_inverse(total, kHidden, args.norm_eps);
     };
     if constexpr (kKB > 1) {
-        // Partial plane kb: this block's sums over its K range, unscaled; the norm's partial
-        // sums of squares per row go after the planes.
+        // Partial plane kb: this block's sums over its K range.
         float* plane = args.split_partials + static_cast<int64_t>(kb) * args.m * args.n;
-        float* plane_ss = args.split_partials + static_cast<int64_t>(kKB) * args.m * args.n +
-                          static_cast<int64_t>(kb) * args.m;
-        if constexpr (kParts == 1) {
 #pragma unroll
-            for (int j = 0; j < kTiles; ++j)
+        for (int r = 0; r < 16; ++r) partial[wave][0][r][lane] = acc[0][r];
+        __syncthreads();
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int64_t out_row = m0 + mfma32_row(lane, r);
-                    if (out_row < args.m) plane[out_row * args.n + n0 + 32 * j + (lane & 31)] = acc[j][r];
-                }
-            if constexpr (kNorm) {
-                if (lane < 32 && m0 + lane < args.m) plane_ss[m0 + lane] = norm_ss[row_tile][lane];
-            }
-        } else {
+        for (int u = 0; u < 16 / kParts; ++u) {
+            const int r = (16 / kParts) * part + u;
+            float v = partial[row_tile][0][r][lane];
 #pragma unroll
-            for (int j = 0; j < kTiles; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) partial[wave][j][r][lane] = acc[j][r];
-            __syncthreads();
-            const int j = lane & 31;
-#pragma unroll
-            for (int u = 0; u < 16 / kParts; ++u) {
-                const int r = (16 / kParts) * part + u;
-                float lo = partial[row_tile][0][r][lane], hi = partial[row_tile][kTiles - 1][r][lane];
-#pragma unroll
-                for (int p = 1; p < kParts; ++p) {
-                    lo += partial[row_tile + RT * p][0][r][lane];
-                    hi += partial[row_tile + RT * p][kTiles - 1][r][lane];
-                }
-                const int64_t out_row = m0 + mfma32_row(lane, r);
-                if (out_row >= args.m) continue;
-                plane[out_row * args.n + n0 + j] = lo;
-                if constexpr (kCols == 64) plane[out_row * args.n + n0 + 32 + j] = hi;
-            }
-            if constexpr (kNorm) {
-                if (part == 0 && lane < 32 && m0 + lane < args.m) {
-                    float total = norm_ss[row_tile][lane];
-#pragma unroll
-                    for (int p = 1; p < kParts; ++p) total += norm_ss[row_tile + RT * p][lane];
-                    plane_ss[m0 + lane] = total;
-                }
-            }
+            for (int p = 1; p < kParts; ++p) v += partial[row_tile + RT * p][0][r][lane];
+            const int64_t out_row = m0 + mfma32_row(lane, r);
+            if (out_row < args.m) plane[out_row * args.n + n0 + (lane & 31)] = v;
         }
     } else if constexpr (kParts == 1 && kCols == 32) {
 #pragma unroll
@@ -492,54 +461,23 @@ __global__ void __launch_bounds__(64 * kRegWaves) gemm_reg_kernel(GemmArgs args)
     }
 }
 
-// Sums the kPlanes partial planes of a K-split gemm_split_kernel or gemm_narrow_kernel in plane order and
-// applies the epilogue: thread -> (row, column pair j / j + 32 of a 64-column group) for
-// kCols = 64, (row, column) for kCols = 32.  The folded norm's row scale comes from the
-// summed partial sums of squares.
-template <GemmEpilogue E, bool kNorm, int kCols, int kPlanes = kSplitBlocksK>
-__global__ void __launch_bounds__(256) gemm_split_reduce_kernel(GemmArgs args) {
-    constexpr bool kPair = kCols == 64;
-    const int units = kPair ? args.n / 2 : args.n;
-    const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= args.m * units) return;
-    const int64_t row = idx / units;
-    const int u = static_cast<int>(idx - row * units);
+// c = residual + (plane 0 + plane 1 + ...): the partial planes of a K-split GEMM (gemm_split_kernel or
+// gemm_limb_kernel) in plane order, thread per output value.
+template <int kPlanes>
+__global__ void __launch_bounds__(256) split_reduce_residual_kernel(GemmArgs args) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     const int64_t plane = args.m * args.n;
-    const float* p = args.split_partials + row * args.n;
-    float inv = 1.0f;
-    if constexpr (kNorm) {
-        const float* ss = args.split_partials + kPlanes * plane + row;
-        float total = ss[0];
+    if (i >= plane) return;
+    float v = args.split_partials[i];
 #pragma unroll
-        for (int b = 1; b < kPlanes; ++b) total += ss[b * args.m];
-        inv = rms_inverse(total, kHidden, args.norm_eps);
-    }
-    if constexpr (kPair) {
-        const int g0 = (u >> 5) * 64;
-        const int j = u & 31;
-        float lo = p[g0 + j], hi = p[g0 + 32 + j];
-#pragma unroll
-        for (int b = 1; b < kPlanes; ++b) {
-            lo += p[b * plane + g0 + j];
-            hi += p[b * plane + g0 + 32 + j];
-        }
-        if constexpr (kNorm) {
-            lo *= inv;
-            hi *= inv;
-        }
-        gemm_store_pair<E>(args, row, g0, j, lo, hi);
-    } else {
-        float v = p[u];
-#pragma unroll
-        for (int b = 1; b < kPlanes; ++b) v += p[b * plane + u];
-        gemm_store_one<E>(args, row, u, v);
-    }
+    for (int b = 1; b < kPlanes; ++b) v += args.split_partials[b * plane + i];
+    args.c[i] = args.residual[i] + v;
 }
 
 // The reduce of a K-split 576-column GEMM with the residual epilogue, folded into the RMSNorm
 // of its output: c = residual + (plane 0 + plane 1 + ...) and norm_out = w * (c * inv_rms(c)).
 // Wave per row, the row in registers as float4 quads; the sums run in the order of
-// gemm_split_reduce_kernel and the norm in that of rmsnorm_wave4_kernel, so both outputs are
+// split_reduce_residual_kernel and the norm in that of rmsnorm_wave4_kernel, so both outputs are
 // bitwise those of the reduce kernel followed by launch_rmsnorm_rows.
 template <int kPlanes>
 __global__ void __launch_bounds__(256) split_reduce_residual_norm_kernel(GemmArgs args, const float* __restrict__ w,
@@ -742,7 +680,7 @@ constexpr int64_t kSplitKBlocks = 256;  // ... and with K split over blocks whil
 constexpr int64_t kNarrowBlocks = 256;
 
 // Tiling of gemm_split_kernel for this GEMM (rt = 0 when it does not take it), for K = 576
-// (hidden) or 1536 (intermediate), while the grid fits the device once.  Plain and residual
+// (hidden) or, plain and residual epilogues, 1536 (intermediate), while the grid fits the device once.  Plain and residual
 // epilogues first try 32-column tiles (one row tile per block).  Otherwise 64-column tiles
 // with the smallest row tiling that fits; shapes the 64 x 64 tile kernel takes use one row
 // tile only: with more, their 9 column tiles leave too many CUs idle (measured slower at
@@ -752,8 +690,8 @@ struct SplitShape {
     int cols;
 };
 static SplitShape split_shape(const GemmArgs& args, GemmEpilogue epilogue) {
-    if (args.k != kHidden && args.k != kInter) return {0, 0};
     const bool plain = epilogue == GemmEpilogue::kStore || epilogue == GemmEpilogue::kResidual;
+    if (args.k != kHidden && !(plain && args.k == kInter)) return {0, 0};
     if (plain && (args.n / 32) * ((args.m + 31) / 32) <= kSplitBlocks) return {1, 32};
     const bool narrow_shape = plain && args.n % 128 != 0 && args.k % 32 == 0;
     for (int rt = 1; rt <= (narrow_shape ? 1 : 4); rt *= 2)
@@ -830,16 +768,15 @@ static hipError_t launch_reg(const GemmArgs& args, GemmEpilogue epilogue, RegSha
     return hipGetLastError();
 }
 
-// True when `parts` partial planes of this GEMM (and as many rows of sums of squares) fit the
-// caller's workspace.
+// True when `parts` partial planes of this GEMM fit the caller's workspace.
 static bool planes_fit(const GemmArgs& args, int parts) {
-    return args.split_partials != nullptr && parts * args.m * (static_cast<int64_t>(args.n) + 1) <= args.split_floats;
+    return args.split_partials != nullptr && parts * args.m * static_cast<int64_t>(args.n) <= args.split_floats;
 }
 
-// Most K parts of a limb GEMM (its partial planes are summed by gemm_split_reduce_kernel or
-// split_reduce_residual_norm_kernel): plain and residual epilogues, as many planes as fit.
+// Most K parts of a limb GEMM (its partial planes are summed by split_reduce_residual_kernel or
+// split_reduce_residual_norm_kernel): residual epilogue, as many planes as fit.
 static int limb_max_parts(const GemmArgs& args, GemmEpilogue epilogue) {
-    if (epilogue != GemmEpilogue::kStore && epilogue != GemmEpilogue::kResidual) return 1;
+    if (epilogue != GemmEpilogue::kResidual) return 1;
     return planes_fit(args, kSplitBlocksK) ? kSplitBlocksK : (planes_fit(args, 2) ? 2 : 1);
 }
 
@@ -850,13 +787,25 @@ static bool narrow_taken(const GemmArgs& args, GemmEpilogue epilogue) {
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-// Whether gemm_split_kernel takes these args with K split over kSplitBlocksK blocks: its grid
-// fits the device once even when tripled, and the caller's planes hold the split.
+// Whether gemm_split_kernel takes these args with K split over kSplitBlocksK blocks: 32-column tiles
+// over the intermediate width whose grid fits the device once even when tripled, and the
+// caller's planes hold the split.
 static bool split_k_taken(const GemmArgs& args, GemmEpilogue epilogue) {
     const SplitShape shape = split_shape(args, epilogue);
-    if (shape.rt == 0) return false;
-    const int64_t blocks = (args.n / shape.cols) * ((args.m + 32 * shape.rt - 1) / (32 * shape.rt));
+    if (epilogue != GemmEpilogue::kResidual || shape.cols != 32 || args.k != kInter) return false;
+    const int64_t blocks = (args.n / 32) * ((args.m + 31) / 32);
     return planes_fit(args, kSplitBlocksK) && blocks * kSplitBlocksK <= kSplitKBlocks;
+}
+
+// c = residual + the sum of `parts` partial planes.
+static hipError_t launch_split_reduce(const GemmArgs& args, int parts, hipStream_t stream) {
+    const dim3 grid(static_cast<unsigned>((args.m * args.n + 255) / 256));
+    if (parts == 2)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(split_reduce_residual_kernel<2>), grid, dim3(256), 0, stream, args);
+    else
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(split_reduce_residual_kernel<kSplitBlocksK>), grid, dim3(256), 0, stream,
+                           args);
+    return hipGetLastError();
 }
 
 static hipError_t gemm_args_valid(const GemmArgs& args, GemmEpilogue epilogue) {
@@ -887,89 +836,53 @@ static hipError_t launch_gemm_split(const GemmArgs& args, GemmEpilogue epilogue,
         const bool hidden = args.k == kHidden;
         dim3 grid(static_cast<unsigned>(args.n / shape.cols), static_cast<unsigned>((args.m + 32 * rt - 1) / (32 * rt)));
         const dim3 split_block(64 * kSplitWaves);
-        // Grids of at most a third of the device split K over kSplitBlocksK blocks when the
-        // caller provides the partial planes.
-        const bool split_k = split_k_taken(args, epilogue);
-        if (split_k) grid.x *= kSplitBlocksK;
-#define FLUX_SPLIT_RT(E, ST, RT, NORM, COLS)                                                                        \
-    do {                                                                                                            \
-        if (split_k)                                                                                                \
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(gemm_split_kernel<E, ST * RT / kSplitBlocksK, RT, NORM, COLS,        \
-                                                                 kSplitBlocksK>),                                   \
-                               grid, split_block, 0, stream, args);                                                 \
-        else                                                                                                        \
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(gemm_split_kernel<E, ST * RT, RT, NORM, COLS, 1>), grid, split_block, \
-                               0, stream, args);                                                                    \
+        if (split_k_taken(args, epilogue)) {
+            grid.x *= kSplitBlocksK;
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(gemm_split_kernel<GemmEpilogue::kResidual, 24 / kSplitBlocksK, 1, false,
+                                                                 32, kSplitBlocksK>),
+                               grid, split_block, 0, stream, args);
+            const hipError_t st = hipGetLastError();
+            return st != hipSuccess ? st : launch_split_reduce(args, kSplitBlocksK, stream);
+        }
+#define FLUX_SPLIT_RT(E, ST, RT, NORM, COLS)                                                                          \
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(gemm_split_kernel<E, ST * RT, RT, NORM, COLS, 1>), grid, split_block, 0, stream, \
+                       args)
+#define FLUX_SPLIT_ROWS(E, ST, NORM)                     \
+    do {                                                 \
+        if (rt == 1) FLUX_SPLIT_RT(E, ST, 1, NORM, 64);      \
+        else if (rt == 2) FLUX_SPLIT_RT(E, ST, 2, NORM, 64); \
+        else FLUX_SPLIT_RT(E, ST, 4, NORM, 64);              \
     } while (0)
-#define FLUX_LAUNCH_SPLIT(E)                                                                            \
-    do {                                                                                                \
-        if (rt == 1) {                                                                                  \
-            if (hidden) FLUX_SPLIT_RT(E, 9, 1, false, 64); else FLUX_SPLIT_RT(E, 24, 1, false, 64);     \
-        } else if (rt == 2) {                                                                           \
-            if (hidden) FLUX_SPLIT_RT(E, 9, 2, false, 64); else FLUX_SPLIT_RT(E, 24, 2, false, 64);     \
-        } else {                                                                                        \
-            if (hidden) FLUX_SPLIT_RT(E, 9, 4, false, 64); else FLUX_SPLIT_RT(E, 24, 4, false, 64);     \
-        }                                                                                               \
+#define FLUX_SPLIT_PLAIN(E)                                             \
+    do {                                                                \
+        if (shape.cols == 32 && hidden) FLUX_SPLIT_RT(E, 9, 1, false, 32); \
+        else if (shape.cols == 32) FLUX_SPLIT_RT(E, 24, 1, false, 32);     \
+        else if (hidden) FLUX_SPLIT_ROWS(E, 9, false);                     \
+        else FLUX_SPLIT_ROWS(E, 24, false);                                \
     } while (0)
-#define FLUX_LAUNCH_SPLIT_PLAIN(E)                                                                      \
-    do {                                                                                                \
-        if (shape.cols == 32) {                                                                         \
-            if (hidden) FLUX_SPLIT_RT(E, 9, 1, false, 32); else FLUX_SPLIT_RT(E, 24, 1, false, 32);     \
-        } else {                                                                                        \
-            FLUX_LAUNCH_SPLIT(E);                                                                       \
-        }                                                                                               \
-    } while (0)
-#define FLUX_LAUNCH_SPLIT_NORM(E)                                                                       \
-    do {                                                                                                \
-        if (rt == 1) FLUX_SPLIT_RT(E, 9, 1, true, 64);                                                  \
-        else if (rt == 2) FLUX_SPLIT_RT(E, 9, 2, true, 64);                                             \
-        else FLUX_SPLIT_RT(E, 9, 4, true, 64);                                                          \
+#define FLUX_SPLIT_PAIR(E)                  \
+    do {                                    \
+        if (norm) FLUX_SPLIT_ROWS(E, 9, true); \
+        else FLUX_SPLIT_ROWS(E, 9, false);     \
     } while (0)
         switch (epilogue) {
             case GemmEpilogue::kStore:
-                FLUX_LAUNCH_SPLIT_PLAIN(GemmEpilogue::kStore);
+                FLUX_SPLIT_PLAIN(GemmEpilogue::kStore);
                 break;
             case GemmEpilogue::kResidual:
-                FLUX_LAUNCH_SPLIT_PLAIN(GemmEpilogue::kResidual);
+                FLUX_SPLIT_PLAIN(GemmEpilogue::kResidual);
                 break;
             case GemmEpilogue::kSwiglu:
-                if (norm) FLUX_LAUNCH_SPLIT_NORM(GemmEpilogue::kSwiglu);
-                else FLUX_LAUNCH_SPLIT(GemmEpilogue::kSwiglu);
+                FLUX_SPLIT_PAIR(GemmEpilogue::kSwiglu);
                 break;
             case GemmEpilogue::kQkvRope:
-                if (norm) FLUX_LAUNCH_SPLIT_NORM(GemmEpilogue::kQkvRope);
-                else FLUX_LAUNCH_SPLIT(GemmEpilogue::kQkvRope);
+                FLUX_SPLIT_PAIR(GemmEpilogue::kQkvRope);
                 break;
         }
-#undef FLUX_LAUNCH_SPLIT_PLAIN
-#undef FLUX_LAUNCH_SPLIT_NORM
-#undef FLUX_LAUNCH_SPLIT
+#undef FLUX_SPLIT_PAIR
+#undef FLUX_SPLIT_PLAIN
+#undef FLUX_SPLIT_ROWS
 #undef FLUX_SPLIT_RT
-        hipError_t st = hipGetLastError();
-        if (st != hipSuccess || !split_k) return st;
-        const int64_t units = shape.cols == 64 ? args.n / 2 : args.n;
-        const dim3 rgrid(static_cast<unsigned>((args.m * units + 255) / 256));
-#define FLUX_REDUCE(E, NORM, COLS) \
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(gemm_split_reduce_kernel<E, NORM, COLS>), rgrid, dim3(256), 0, stream, args)
-        switch (epilogue) {
-            case GemmEpilogue::kStore:
-                if (shape.cols == 32) FLUX_REDUCE(GemmEpilogue::kStore, false, 32);
-                else FLUX_REDUCE(GemmEpilogue::kStore, false, 64);
-                break;
-            case GemmEpilogue::kResidual:
-                if (shape.cols == 32) FLUX_REDUCE(GemmEpilogue::kResidual, false, 32);
-                else FLUX_REDUCE(GemmEpilogue::kResidual, false, 64);
-                break;
-            case GemmEpilogue::kSwiglu:
-                if (norm) FLUX_REDUCE(GemmEpilogue::kSwiglu, true, 64);
-                else FLUX_REDUCE(GemmEpilogue::kSwiglu, false, 64);
-                break;
-            case GemmEpilogue::kQkvRope:
-                if (norm) FLUX_REDUCE(GemmEpilogue::kQkvRope, true, 64);
-                else FLUX_REDUCE(GemmEpilogue::kQkvRope, false, 64);
-                break;
-        }
-#undef FLUX_REDUCE
         return hipGetLastError();
     }
     const int max_parts = limb_max_parts(args, epilogue);
@@ -986,20 +899,7 @@ static hipError_t launch_gemm_split(const GemmArgs& args, GemmEpilogue epilogue,
     const LimbPlan plan = limb_plan(args, max_parts, false);
     const hipError_t st = launch_limb_gemm(args, epilogue, plan, stream);
     if (st != hipSuccess || plan.parts == 1) return st;
-    const dim3 rgrid(static_cast<unsigned>((args.m * args.n + 255) / 256));
-#define FLUX_REDUCE_PLAIN(P)                                                                                        \
-    do {                                                                                                            \
-        if (epilogue == GemmEpilogue::kResidual)                                                                    \
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(gemm_split_reduce_kernel<GemmEpilogue::kResidual, false, 32, P>),    \
-                               rgrid, dim3(256), 0, stream, args);                                                  \
-        else                                                                                                        \
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(gemm_split_reduce_kernel<GemmEpilogue::kStore, false, 32, P>), rgrid, \
-                               dim3(256), 0, stream, args);                                                         \
-    } while (0)
-    if (plan.parts == 2) FLUX_REDUCE_PLAIN(2);
-    else FLUX_REDUCE_PLAIN(kSplitBlocksK);
-#undef FLUX_REDUCE_PLAIN
-    return hipGetLastError();
+    return launch_split_reduce(args, plan.parts, stream);
 }
 
 hipError_t launch_norm_gemm(const GemmArgs& args, const float* norm_weight, float eps, float* scratch,

@@ -11,14 +11,6 @@ namespace {
 constexpr int kLimbStage = 16;   // K values per stage
 constexpr int kLimbBN = 128;     // block columns: two waves of 64 (one epilogue column group each)
 
-template <int S, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (S < N) {
-        f(std::integral_constant<int, S>{});
-        static_for<S + 1, N>(f);
-    }
-}
-
 // C = epilogue(A[M,K] * W[N,K]^T).  Block tile (32 TM WM) x 128, WM x 2 waves, wave tile
 // (32 TM) x 64.
 //

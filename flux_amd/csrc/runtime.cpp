@@ -558,11 +558,8 @@ PrefillRuntime::PrefillRuntime(const flux_weights& weights, const float* rope_co
     const size_t o_attn = take(sizeof(float) * s * kHidden);
     const size_t o_swiglu = take(sizeof(float) * s * kInter);
     const size_t o_attn_ws = take(sizeof(float) * prefill_attention_workspace_floats(s));
-    // Partial planes of the K-split GEMMs, whose grids are small only for short and mid-length
-    // prompts: sized for gate/up up to kSplitKMaxRows rows, for the 576-column GEMMs beyond.
-    const bool split_k = s <= kNarrowSplitMaxRows;
-    const int64_t split_n = s <= kSplitKMaxRows ? kGateUp : kHidden;
-    const size_t o_split = take(split_k ? sizeof(float) * split_partials_floats(s, split_n) : 0);
+    // Partial planes of the K-split GEMMs (o_proj and down).
+    const size_t o_split = take(sizeof(float) * split_partials_floats(s, kHidden));
     const size_t o_final = take(sizeof(float) * kHidden);
     const size_t o_logits = take(sizeof(float) * vocab_);
     const size_t o_token = take(sizeof(int64_t));
@@ -581,8 +578,8 @@ PrefillRuntime::PrefillRuntime(const flux_weights& weights, const float* rope_co
     attn_rows_ = reinterpret_cast<float*>(base + o_attn);
     swiglu_ = reinterpret_cast<float*>(base + o_swiglu);
     attn_workspace_ = reinterpret_cast<float*>(base + o_attn_ws);
-    split_partials_ = split_k ? reinterpret_cast<float*>(base + o_split) : nullptr;
-    split_floats_ = split_k ? split_partials_floats(s, split_n) : 0;
+    split_partials_ = reinterpret_cast<float*>(base + o_split);
+    split_floats_ = split_partials_floats(s, kHidden);
     final_hidden_ = reinterpret_cast<float*>(base + o_final);
     logits_ = reinterpret_cast<float*>(base + o_logits);
     initial_token_ = reinterpret_cast<int64_t*>(base + o_token);
@@ -645,8 +642,6 @@ void PrefillRuntime::run(const int64_t* input_ids, hipStream_t stream) {
         float* keys = db.key_cache + layer * layer_elems;
         float* values = db.value_cache + layer * layer_elems;
         GemmArgs qkv{};
-        qkv.split_partials = split_partials_;
-        qkv.split_floats = split_floats_;
         qkv.b = weights_.packed_qkv[layer];
         qkv.m = seq_;
         qkv.n = kQKV;
@@ -680,8 +675,6 @@ void PrefillRuntime::run(const int64_t* input_ids, hipStream_t stream) {
         o.n = kHidden;
         o.k = kHidden;
         GemmArgs gu{};
-        gu.split_partials = split_partials_;
-        gu.split_floats = split_floats_;
         gu.b = weights_.gate_up[layer];
         gu.c = swiglu_;
         gu.m = seq_;

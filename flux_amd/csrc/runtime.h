@@ -156,7 +156,7 @@ private:
     float* query_ = nullptr;      // [9, S, 64]
     float* attn_rows_ = nullptr;  // [S, 576]
     float* attn_workspace_ = nullptr;  // split-key attention partials
-    float* split_partials_ = nullptr;  // K-split GEMM partial planes (short prompts), or null
+    float* split_partials_ = nullptr;  // partial planes of the K-split o_proj and down GEMMs
     int64_t split_floats_ = 0;         // floats at split_partials_
     float* swiglu_ = nullptr;     // [S, 1536]
     float* final_hidden_ = nullptr;  // [576]
