@@ -250,10 +250,9 @@ def test_mfma_linear(gpu_device, m, n, k):
     # k = 576 with at most 256 16-row tiles: the register kernel, 32 columns wide (16, 200 rows)
     # or 64 (130 rows).  Otherwise k = 576 or 1536 with at most 256 tiles: the split kernel, on
     # 32 x 32 tiles (257 rows), else on (32 RT) x 64 tiles with RT = 1 (512 rows), 2 (600 rows)
-    # or 4 (1200 rows); widths that are not a multiple of 128 only with RT = 1. Otherwise those
-    # widths take the 64 x 64 tile kernel when k % 32 == 0 (1000, 2048 rows), else the
-    # 128-column kernel; grids under 256 blocks take their four-buffer ring variants (300 rows
-    # with k = 64, 1000 rows, and the first three cases).
+    # or 4 (1200 rows); widths that are not a multiple of 128 only with RT = 1.  Otherwise the
+    # 64 x 64 tile kernel while k % 32 == 0 and at most 256 tiles (64 and 1000 rows, both of 300),
+    # else three-limb products (1, 70, 1024 and 2048 rows).
     a = _randn(m, k, seed=61).to(gpu_device)
     w = _randn(n, k, seed=62, std=0.05).to(gpu_device)
     r = _randn(m, n, seed=63).to(gpu_device)

@@ -17,6 +17,10 @@ def _randn(*shape, seed, std=1.0):
     return (torch.randn(*shape, generator=torch.Generator().manual_seed(seed)) * std).float()
 
 
+def _rel(got, want):
+    return float((got - want).norm() / want.norm())
+
+
 def _linear(a, w, residual, device):
     m, k = a.shape
     n = w.shape[0]
@@ -32,8 +36,8 @@ def _linear(a, w, residual, device):
 @pytest.mark.parametrize("m,n,k", [
     (1, 64, 16), (65, 192, 48),          # one stage; an odd number of stages, a half-empty column tile
     (1793, 576, 576), (2049, 576, 1536),  # 64-row tiles, the last of one row
-    (1025, 3072, 64), (3073, 960, 576),   # 128-row tiles
-    (8193, 3072, 32),                     # 256-row tiles
+    (1025, 3072, 64), (3073, 960, 576), (8193, 3072, 32),  # 128-row tiles
+    (7937, 3072, 32), (2501, 3072, 576),  # 256-row tiles, the last of one row and of 197
 ])
 def test_limb_linear_error_bound(gpu_device, m, n, k):
     a, w, r = _randn(m, k, seed=1), _randn(n, k, seed=2, std=0.05), _randn(m, n, seed=3)
@@ -41,14 +45,22 @@ def test_limb_linear_error_bound(gpu_device, m, n, k):
     size = a.double().abs() @ w.double().abs().T
     # Each limb product is exact.  The leading limbs' accumulator is rounded once per 16 K values
     # at no more than the size of the sum of magnitudes, the small products' five times as often
-    # at 2^-8 of it; the dropped products are below 2^-25 of it.  Two units in the last place per
-    # rounding leave room for an instruction that truncates what it adds up.
+    # at 2^-8 of it; the dropped products are below 2^-23 of it (a second times a third limb, twice,
+    # of at most 2^-8 and 2^-16 of their values).  Two units in the last place per rounding leave
+    # room for an instruction that truncates what it adds up.
     bound = size * (k / 16 * (1 + 5 / 256) + 2) * 2.0 ** -22
+    # In the norm: a rounding error is 2^-24 / sqrt(3) of what is rounded, and the partial sums of
+    # random products grow as the root of their number, so K / 16 of them add up to
+    # sqrt(K / 32) of that; half as much again, and one for the last rounding.  Without the third
+    # limb the error is about ten times this bound.
+    norm = (1.5 * math.sqrt(k / 32) + 1) * 2.0 ** -24 / math.sqrt(3)
     for residual in (None, r):
         c = _linear(a, w, residual, gpu_device).double()
         want = exact if residual is None else exact + r.double()
         limit = bound if residual is None else bound + want.abs() * 2.0 ** -23
         assert torch.all((c - want).abs() <= limit)
+        if residual is None and k >= 576:
+            assert _rel(c, want) < norm
 
 
 def test_limb_linear_keeps_float32_range(gpu_device):
@@ -67,13 +79,13 @@ def test_limb_linear_keeps_float32_range(gpu_device):
     assert torch.equal(c[4], -torch.sign(w[:, 9]) * float("inf"))
     assert torch.all(torch.isnan(c[5]))
     torch.testing.assert_close(c[6].double(), 3.4e38 * w[:, 2].double(), rtol=1e-6, atol=0)
-    torch.testing.assert_close(c[700].double(), a[700].double() @ w.double().T, rtol=0, atol=1e-42 * k)
+    # Float32 rounds K / 2 sums of two products to multiples of 2^-149, by at most half of one, and
+    # the result and the products once more; the outputs are thousands of them.
+    want = a[700].double() @ w.double().T
+    torch.testing.assert_close(c[700].double(), want, rtol=0, atol=k * 2.0 ** -149)
+    assert torch.all(c[700][want.abs() > k * 2.0 ** -149] != 0.0) and float(want.abs().max()) > 10 * k * 2.0 ** -149
     rows = [r for r in range(m) if r not in (3, 4, 5, 6, 700)]
     torch.testing.assert_close(c[rows].double(), a[rows].double() @ w.double().T, rtol=1e-4, atol=1e-4)
-
-
-def _rel(got, want):
-    return float((got - want).norm() / want.norm())
 
 
 def _rows_call(name, x, w, device):
@@ -101,6 +113,19 @@ def _rows_call(name, x, w, device):
         want = torch.cat((heads[:12] + paired.float() * 0.0, heads[12:]))
     torch.cuda.synchronize()
     return out.cpu(), want
+
+
+@pytest.mark.parametrize("name,n", [("linear", 576), ("gate_up", 3072), ("qkv", 960)])
+def test_limb_gemm_infinity_and_nan(gpu_device, name, n):
+    # An infinity in one row and a NaN in another, in different tiles; all others as without.
+    x, w = _randn(2500, 576, seed=34), _randn(n, 576, seed=35, std=0.05)
+    x[3, 7], x[2499, 11] = float("inf"), float("nan")
+    got, want = _rows_call(name, x, w, gpu_device)
+    want = want.float()
+    odd = ~torch.isfinite(want)
+    assert int(odd.sum()) == 2 * (want.shape[-1] if name != "qkv" else 960)
+    torch.testing.assert_close(got[odd], want[odd], rtol=0, atol=0, equal_nan=True)
+    torch.testing.assert_close(got[~odd], want[~odd], rtol=5e-4, atol=1e-4)
 
 
 # 2500 rows: the limb kernel under each epilogue.
@@ -203,6 +228,25 @@ def test_limb_attention_keeps_float32_range(gpu_device):
     assert torch.all(got[6:, 1000:, 5] == float("inf"))
     rest = [d for d in range(64) if d != 5]
     torch.testing.assert_close(got[6:, :, rest], want[6:, :, rest], rtol=2e-4, atol=2e-5)
+
+
+def test_limb_attention_nan(gpu_device):
+    # A NaN key or value reaches every query that sees its row, a NaN query its own row only.
+    seq = 1500
+    q, k, v = _randn(9, seq, 64, seed=37), _randn(3, seq, 64, seed=38), _randn(3, seq, 64, seed=39)
+    want = _attention64(q, k, v)
+    k[0, 1200, 3] = float("nan")
+    v[1, 1300, 4] = float("nan")
+    q[8, 70, 5] = float("nan")
+    got = _attention(q, k, v, gpu_device)
+    assert torch.all(torch.isnan(got[:3, 1200:])) and torch.all(torch.isnan(got[3:6, 1300:, 4]))
+    assert torch.all(torch.isnan(got[8, 70]))
+    seen = torch.ones(9, seq, 64, dtype=torch.bool)
+    seen[:3, 1200:] = False
+    # Masked weights are exactly zero, and zero times NaN is NaN: the value's 64-key tile too.
+    seen[3:6, 1280:, 4] = False
+    seen[8, 70] = False
+    torch.testing.assert_close(got[seen], want[seen], rtol=2e-4, atol=2e-5)
 
 
 def test_limb_attention_overflow_is_infinite(gpu_device):

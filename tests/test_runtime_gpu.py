@@ -457,17 +457,17 @@ def test_prefill_input_errors(small_model):
         native.prefill(ids[:, :-1])
 
 
-@pytest.mark.parametrize("length", [1, 7, 9, 45, 333, 512, 513, 1024, 1025, 1537, 3001])
+@pytest.mark.parametrize("length", [1, 7, 9, 45, 112, 113, 129, 273, 333, 512, 513, 897, 1024, 1025, 1537, 3001])
 def test_odd_length_prefill_matches_oracle(small_model, length):
     """Prompt lengths that end inside a 128-query attention tile and split the keys of the
-    later tiles into chunks (333: 2-tile, 1537: 4-tile, 3001: 8-tile chunks), through the whole
+    later tiles into chunks (513: 2-tile, 1537: 6-tile, 3001: 12-tile chunks), through the whole
     native prefill, against the CPU oracle: last-row logits, greedy token, K/V cache rows.
     Short prompts also take the GEMMs that fold the RMSNorm (1, 7, 9 and 45 rows end inside
-    the first 16-row tile of the register kernel or 32-row tile of the split kernel).  1 | 7 | 9:
-    up to 8 rows the next layer's QKV kernel sums the down GEMM's partial planes and residual
-    (no reduce kernel), 9 rows take the reduce.  512 | 513 straddle the one-kernel
-    attention's limit (512 tokens), and 1024 | 1025 the limit up to which the K-split planes
-    are sized for gate/up (1024 rows), so both sides of each switch run."""
+    the first 16-row tile of the register kernel or 32-row tile of the split kernel).
+    112 | 113: the down GEMM on register tiles, then on K thirds (129: on all of K); 273: the
+    first QKV on the split kernel; 512 | 513 straddle the one-kernel attention's limit, 897 is the
+    first prompt of limb attention and of o_proj and down on limb tiles (64 rows, three K planes),
+    1537 takes two planes and 3001 128-row tiles."""
     g = torch.Generator().manual_seed(length)
     prompt = torch.randint(0, 128, (1, length), generator=g)
     runtime = NativeSmolLM2Prefill.capture(small_model, prompt.cuda(), max_decode_steps=1)
@@ -612,3 +612,73 @@ def test_decode_across_the_single_chunk_limit(small_model):
             torch.testing.assert_close(decoded, reference.logits[0, 0].float().cpu(), atol=LOGIT_ATOL, rtol=LOGIT_RTOL,
                                        msg=lambda m: f"{n_prompt} + {step}: {m}")
         assert runtime.device_error() == 0
+
+
+def _layer0_float64(state, prompt):
+    """The K and V rows of layer 1 (before RoPE of K) of a prompt, in float64 from float32 weights."""
+    w = {k: v.double().cuda() for k, v in state.items() if k.startswith(("model.embed", "model.layers.0.", "model.layers.1."))}
+
+    def norm(x, weight):
+        return weight * (x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-5))
+
+    def rotate(x):
+        n = x.shape[1]
+        inv = 1.0 / (synthetic.ROPE_THETA ** (torch.arange(0, 64, 2, dtype=torch.float32) / 64))
+        angle = (torch.arange(n, dtype=torch.float32)[:, None] * inv[None]).repeat(1, 2)
+        c, s = angle.cos().double().cuda(), angle.sin().double().cuda()
+        return x * c + torch.cat((-x[..., 32:], x[..., :32]), -1) * s
+
+    n = prompt.shape[1]
+    p = "model.layers.0."
+    h = w["model.embed_tokens.weight"][prompt[0].cuda()]
+    x = norm(h, w[p + "input_layernorm.weight"])
+    q, k, v = ((x @ w[p + f"self_attn.{c}_proj.weight"].T).view(n, -1, 64).transpose(0, 1) for c in "qkv")
+    q, k = rotate(q), rotate(k)
+    out = torch.empty(n, 576, dtype=torch.float64, device="cuda")
+    future = torch.ones(n, n, dtype=torch.bool, device="cuda").triu(1)
+    for head in range(9):
+        scores = (q[head] @ k[head // 3].T * 0.125).masked_fill_(future, float("-inf"))
+        out[:, 64 * head:64 * head + 64] = torch.softmax(scores, -1) @ v[head // 3]
+    h = h + out @ w[p + "self_attn.o_proj.weight"].T
+    x = norm(h, w[p + "post_attention_layernorm.weight"])
+    gate = x @ w[p + "mlp.gate_proj.weight"].T
+    h = h + (gate / (1 + torch.exp(-gate)) * (x @ w[p + "mlp.up_proj.weight"].T)) @ w[p + "mlp.down_proj.weight"].T
+    x = norm(h, w["model.layers.1.input_layernorm.weight"])
+    k, v = ((x @ w[f"model.layers.1.self_attn.{c}_proj.weight"].T).view(n, 3, 64).transpose(0, 1) for c in "kv")
+    return rotate(k), v
+
+
+# o_proj and down on K planes: 3 and 3 on 64-row tiles, 2 on 64 and 3 on 128, 3 on 128, 3 on 256, 2 on 256.
+@pytest.mark.parametrize("length", [1000, 1100, 1700, 3300, 4400])
+def test_prefill_plane_sums_are_as_exact_as_float32(small_model, length):
+    """What layer 0 hands on: sums of 576 and 1536 products in two or three planes, against float64.  Seven
+    contractions and norms of a few 1e-7 each; products without a third limb are 3.5e-6 off."""
+    g = torch.Generator().manual_seed(length)
+    prompt = torch.randint(0, 128, (1, length), generator=g)
+    runtime = NativeSmolLM2Prefill.capture(small_model, prompt.cuda(), max_decode_steps=0)
+    torch.cuda.synchronize()
+    state = synthetic.synthetic_state_dict(synthetic.SyntheticSpec(seed=2701, vocab=128))
+    for got, want in zip((runtime.key_cache[1, 0], runtime.value_cache[1, 0]), _layer0_float64(state, prompt)):
+        error = float((got[:, :length].double() - want).norm() / want.norm())
+        assert error < 1e-6, error
+
+
+@pytest.mark.parametrize("length", [1000, 1100, 4400])
+def test_prefill_planes_keep_float32_range(small_model, length):
+    """An o_proj weight above the largest bf16: its partial planes are those of the float32 instruction, and the
+    hidden rows so large that their squares overflow, so that every norm after them is zero and not NaN."""
+    weight = small_model.model.layers[0].self_attn.o_proj.weight
+    g = torch.Generator().manual_seed(length)
+    prompt = torch.randint(0, 128, (1, length), generator=g)
+    before = weight[5, 7].clone()
+    try:
+        with torch.no_grad():
+            weight[5, 7] = 3.4e38
+        runtime = NativeSmolLM2Prefill.capture(small_model, prompt.cuda(), max_decode_steps=0)
+        torch.cuda.synchronize()
+        assert torch.all(runtime.key_cache[1:, :, :, :length] == 0.0)
+        assert torch.all(runtime.value_cache[1:, :, :, :length] == 0.0)
+        assert torch.all(runtime.logits == 0.0)
+    finally:
+        with torch.no_grad():
+            weight[5, 7] = before
