@@ -42,10 +42,10 @@ namespace {
 // barrier.
 //
 // Bound by power, as the limb GEMMs: 8192 tokens 632 -> 405 us with the planes and the merge
-// (191 TFLOP/s of float32 products, 1.15 PFLOP/s of bf16), 4096: 185 -> 117, 2048: 64 -> 47,
-// 1024: 30.6 -> 27.5; the error against 64 bits at 8000 tokens 4.3e-7 -> 1.7e-7.  Blocks whose
-// values limbs cannot hold, and prompts below kLimbAttnMinSeq, take the float32 instruction
-// (attention_item_f32).
+// (191 TFLOP/s of float32 products, 1.15 PFLOP/s of bf16; 401 to 429 from card to card), 4096:
+// 185 -> 118, 2048: 64 -> 48.7, 1024: 30.6 -> 29.1; the error against 64 bits at 8000 tokens
+// 4.3e-7 -> 1.7e-7.  Blocks whose values or sums limbs cannot hold (kLimbMaxScore and what follows
+// it), and prompts below kLimbAttnMinSeq, take the float32 instruction (attention_item_f32).
 constexpr int kQTile = 128;
 constexpr int kKTile = 64;
 constexpr int kAttnThreads = 256;
@@ -153,7 +153,8 @@ constexpr int kKTileWords = kKTile * kKRow;           // 4352
 constexpr int kKCopies = kKTileWords / 256;           // 17 global_load_lds of 1 KB
 constexpr int kVCopies = kKVTileFloats / 256;         // 16
 
-// One block's item on the float32 instruction, for values that limbs cannot hold.
+// One block's item on the float32 instruction: every block of a prompt below kLimbAttnMinSeq, and
+// blocks of longer ones whose values limbs cannot hold.
 __device__ __forceinline__ void attention_item_f32(const float* __restrict__ q, const float* __restrict__ key_cache,
                                                 const float* __restrict__ value_cache, int64_t seq, int64_t capacity,
                                                 float scale, float* __restrict__ workspace,

@@ -675,8 +675,8 @@ constexpr int64_t kSplitKBlocks = 256;  // ... and with K split over blocks whil
 // what is left then without partial planes, e.g. one layer's o_proj up to 1792 rows: a limb block
 // is longer than one of its blocks there (1000 rows, K = 576: 21 against 13 us; K = 1536, 1536
 // rows: 49 against 31; 500 x 1024, K = 64: 6.2 against 4.9, K = 1024: 33 against 20), and shorter
-// beyond (2048 rows: 21 against 25; 49 against 57).  Only below K = 128 is it even with limb
-// tiles on two rounds of blocks.
+// beyond (2048 rows: 21 against 25; 49 against 57).  On two rounds of blocks it is
+// even with limb tiles at K = 64 and 128 at best.
 constexpr int64_t kNarrowBlocks = 256;
 
 // Tiling of gemm_split_kernel for this GEMM (rt = 0 when it does not take it), for K = 576

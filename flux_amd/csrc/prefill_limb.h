@@ -2,13 +2,14 @@
 //
 // A float32 value is the exact sum of three bf16 limbs (8 + 8 + 8 significant bits, each
 // rounded to nearest from what the limbs before it leave), so a product of two values is nine
-// limb products.  The six largest are kept: the dropped three are below 2^-26 of the product,
-// less than the rounding of one float32 addition.  Each limb product is exact in float32 and
-// v_mfma_f32_32x32x16_bf16 sums sixteen of them per instruction, against two per
-// v_mfma_f32_32x32x2_f32, so the accumulator is rounded less often and the result is, if
-// anything, closer to the exact sum (normal data, K = 576: 3.6e-7 against 4.4e-7 relative;
-// K = 1536: 6.0e-7 against 6.8e-7).  Six of these instructions take 192 cycles for sixteen K
-// values, eight of the float32 ones 512.
+// limb products.  The six largest are kept: the dropped three are at most 2^-23 of the product
+// (a second times a third limb, twice), and 5.7e-9 of a sum of random ones.  Each limb product is
+// exact in float32 and v_mfma_f32_32x32x16_bf16 sums sixteen of them per instruction, against
+// two per v_mfma_f32_32x32x2_f32, so the accumulator is rounded less often and, with the small
+// products in an accumulator of their own, the result is closer to the exact sum (normal data,
+// K = 576: 1.4e-7 against 4.3e-7 relative; 1536: 2.3e-7 against 7.0e-7; 4096: 4.0e-7 against
+// 1.15e-6).  Six of these instructions take 192 cycles for sixteen K values, eight of the
+// float32 ones 512.
 //
 // That holds from 2^-110 to the largest bf16.  Limbs cannot carry infinities (inf - inf) nor
 // magnitudes above (kLimbMax), bf16 has no bits below 2^-133 for the low limbs of smaller values

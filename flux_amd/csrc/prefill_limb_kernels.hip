@@ -28,9 +28,10 @@ constexpr int kLimbBN = 128;     // block columns: two waves of 64 (one epilogue
 // the matrix cores busy while the waves of a SIMD run the same code in step (8192 x 3072 x 576:
 // 164 us, 175 without them).
 //
-// Bound by power: 8192 x 3072 x 576 takes 160 us (181 TFLOP/s of float32 products, 1.09 PFLOP/s
-// of bf16; a large bf16 matrix product reaches 1.18 on this card), and 110 when every value is
-// zero.  The float32 instruction took 228 us there.  A second accumulator for the small
+// Bound by power: 8192 x 3072 x 576 takes 152 to 170 us from card to card (170 to 190 TFLOP/s of
+// float32 products, 1.02 to 1.14 PFLOP/s of bf16; a large bf16 matrix product reaches 1.18), at
+// 1.9 GHz with the matrix cores busy for half of it, and 110 when every value is zero.  The
+// float32 instruction took 228 us there.  A second accumulator for the small
 // products costs 6% of the time and takes the error against 64 bits from 3.6e-7 to 1.4e-7 at
 // K = 576 (float32 instruction: 4.4e-7).
 //
@@ -283,7 +284,8 @@ __global__ void __launch_bounds__(128 * WM, 2) gemm_limb_kernel(GemmArgs args) {
 }
 
 // Microseconds per stage of a grid of `blocks` blocks (fits of measured times, 24 to 3072 blocks
-// at K = 576): one round of 256 x 128 tiles (8 waves, one block per CU) takes 1.0 to 1.5 as it
+// at K = 576; at K = 64 to 4096 and widths of 576 to 3072 the tile chosen by them measured within
+// 8% of the fastest, most within 2%): one round of 256 x 128 tiles (8 waves, one block per CU) takes 1.0 to 1.5 as it
 // fills, 256 blocks of 128 x 128 (two per CU) 0.73 to 0.9 alone and 0.8 each beyond, 256 of
 // 64 x 128 0.46 each and never under 0.57.
 double stage_us(int rows, int64_t blocks) {

@@ -354,8 +354,8 @@ int flux_greedy_argmax_update_f32(const float* logits, int64_t vocab, int64_t* i
                                   int64_t* generation_step, int64_t generated_capacity, int64_t* position,
                                   const int64_t* attention_length, hipStream_t stream);
 
-/* Prefill linear (FP32 MFMA, or bf16 MFMA on three-limb operands at large sizes): C[m,n] = A[m,k] W[n,k]^T
- * (+ residual[m,n]).
+/* Prefill linear (FP32 MFMA, or bf16 MFMA on three-limb operands at large sizes, where a tile whose
+ * values limbs do not carry exactly enough takes FP32 MFMA): C[m,n] = A[m,k] W[n,k]^T (+ residual[m,n]).
  * Replaces linear_fp32 / cublasSgemm (native_prefill_runtime_cuda.cu:285-302).
  * n % 64 == 0, k % 16 == 0. */
 int flux_linear_f32(const float* a, const float* weight, const float* residual, float* c, int64_t m, int64_t n,
@@ -380,7 +380,8 @@ int flux_qkv_rope_cache_rows_f32(const float* x, const float* packed_qkv, const 
 int flux_prefill_attention_workspace_bytes(int64_t seq, int64_t* bytes);
 
 /* Causal GQA prefill attention (FP32 MFMA, or bf16 MFMA on three-limb operands from
- * 897 tokens on; online softmax, keys split in chunks of 128 to 2048 and merged): q [9,seq,64], K/V [3,capacity,64] -> out_rows [seq, 576].
+ * 897 tokens on; online softmax, keys split in chunks of 128 to 2048 and merged):
+ * q [9,seq,64], K/V [3,capacity,64] -> out_rows [seq, 576].
  * `workspace` may be NULL when flux_prefill_attention_workspace_bytes reports 0.
  * Every pointer must be 16-byte aligned.
  * Replaces streaming_prefill_gqa_cuda_fp32 (csrc/streaming_prefill_gqa/
