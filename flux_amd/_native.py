@@ -258,11 +258,13 @@ def ptr(tensor: torch.Tensor | None) -> int | None:
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def current_stream(device: torch.device | None = None) -> int:
-    if _raw_stream is None:
-        return int(torch.cuda.current_stream(device).cuda_stream)
-    index = None if device is None else device.index
-    return int(_raw_stream(torch.cuda.current_device() if index is None else index))
+def current_stream(device: torch.device | int | str | None = None) -> int:
+    if _raw_stream is not None:
+        if device is None:
+            return int(_raw_stream(torch.cuda.current_device()))
+        if isinstance(device, torch.device) and device.type == "cuda":
+            return int(_raw_stream(torch.cuda.current_device() if device.index is None else device.index))
+    return int(torch.cuda.current_stream(device).cuda_stream)
 
 
 class _DeviceArray:

@@ -70,6 +70,23 @@ def test_missing_native_library_fails_loudly(monkeypatch):
         smollm2_flux.enable_flux_ops(_model())
 
 
+@pytest.mark.parametrize("device,raw", [(None, 7), (torch.device("cuda"), 7), (torch.device("cuda:1"), 1), (1, None),
+                                        ("cuda:1", None), (torch.device("cpu"), None)])
+def test_current_stream_takes_what_torch_takes(monkeypatch, device, raw):
+    """Indices, texts and devices of another type go to torch, which resolves or refuses them."""
+    from flux_amd import _native
+
+    class Stream:
+        cuda_stream = 99
+
+    asked = []
+    monkeypatch.setattr(_native, "_raw_stream", lambda index: 1000 + index)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 7)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: asked.append(d) or Stream())
+    assert _native.current_stream(device) == (99 if raw is None else 1000 + raw)
+    assert asked == ([device] if raw is None else [])
+
+
 def test_packed_parameters_and_equivalence():
     reference = _model()
     flux = _model()
